@@ -5,11 +5,10 @@
 // every conv route of vk_engine.cpp:578-608 (1x1 GEMM, Winograd, im2col + GEMM):
 //   * A_DENSE: A is row-major [M, lda]; columns [K1, K) may come from a second
 //     source (the 1x1 shortcut over the up-path concat, vk_engine.cpp:634, :754).
-//   * A_CONV3: A is the implicit im2col of an NHWC image for a 3x3 conv, pad 1,
-//     stride 1/2 (downsample, :689-692), optional nearest-2x upsample folded into
-//     the index math (upsample, :693-697).  K index = tap*Cin + ci.  Columns past
-//     9*Cin may come from one or two dense sources of the same pixels: a resnet's
-//     1x1 shortcut (:634) summed into its conv2.
+//   * A_CONV3: A is the implicit im2col of an NHWC image for a 3x3 conv, pad 1, for the
+//     convs the patch-resident kernel (k_conv.hip) does not take: stride 2 (downsample,
+//     :689-692), nearest-2x upsample folded into the index math (upsample, :693-697), or
+//     channel counts outside its multiples.  K index = tap*Cin + ci.
 // Epilogue (fused; the reference runs these as separate AB/AB2/ADD/GEGLU passes):
 // + bias[n] + bias2[n] (fp32 time projection), GEGLU over interleaved a/b column
 // blocks, + residual, activation (ReLU / quick-GELU), store fp16 / fp32 / fp32-NCHW.  A LayerNorm (layernorm_f32.comp,
@@ -19,7 +18,7 @@
 // with the LayerNorm's affine folded into its W and bias.
 // Split-K, two ways: the last block of a tile to arrive sums the tile's fp32 partials
 // and runs the epilogue (few splits), or a reduce kernel does (many splits).
-#include "sdu_internal.h"
+#include "gemm_common.h"
 
 #include <cstdio>
 
@@ -27,10 +26,7 @@
 
 namespace sdu {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 
 // Final value for output element (m, output column nout) given the fp32 GEMM
@@ -60,62 +56,13 @@ __device__ __forceinline__ void epi_store(const GemmArgs& a, int m, int n, float
 // All-zero 16-byte source for DMA lanes outside the operands (conv padding, K tail).
 __device__ __attribute__((aligned(64))) uint4 g_zero_page[4];
 
-// s_waitcnt vmcnt(N) lgkmcnt(0): at most N vector-memory ops (the DMA of later
-// tiles) outstanding, and every LDS read of this wave complete, so that after the
-// following barrier no wave still reads the ring stage the next DMA overwrites.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt_lgkm0() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0x0 << 8) | ((N >> 4) << 14));
-}
-
-// The same with the tiles issued after the one about to be read still in flight: at
+// wait_vmcnt_lgkm0 with the tiles issued after the one about to be read still in flight: at
 // most `ahead` (<= A) tiles of LPT DMA instructions each.
 template <int LPT, int A>
 __device__ __forceinline__ void wait_tiles(int ahead) {
     if constexpr (A == 0) wait_vmcnt_lgkm0<0>();
     else if (ahead >= A) wait_vmcnt_lgkm0<A * LPT>();
     else wait_tiles<LPT, A - 1>(ahead);
-}
-
-// Sum the per-thread column statistics of a block over the threads that own the same
-// 8 columns (thread t owns chunk t % CPR; chunk c covers columns col0 + 8c ..) through
-// LDS and add them to the per-(image, channel) fp64 statistics, one atomic per value,
-// the sums spread over all threads (each one's NTH / CPR LDS reads issued together).
-// red must hold NTH * 32 floats and be free (the caller's last LDS use is complete
-// after the first barrier here).  Value v of thread t sits at v * NTH + (t ^ v): the
-// stores (one v, consecutive t) and the loads (consecutive v, one t) both fall on
-// distinct banks (a thread-major layout, 32 floats per thread, put every lane of a
-// store on one bank).
-template <int NTH, int CPR>
-__device__ __forceinline__ void stats_flush(const GemmArgs& a, const float (&st)[2][2][8], int b0,
-                                            int m_last, int col0, float* red) {
-    static_assert(NTH % 32 == 0, "swizzle stays within a row");
-    const int tid = threadIdx.x;
-    __syncthreads();
-#pragma unroll
-    for (int sl = 0; sl < 2; ++sl)
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int v = sl * 16 + q * 8 + e;
-                red[v * NTH + (tid ^ v)] = st[sl][q][e];
-            }
-    __syncthreads();
-    const int nslot = m_last / a.stats_hw != b0 ? 2 : 1;
-    // value v of chunk c: slot v / 16, sum (0) or sum of squares (1) = (v / 8) % 2, column v % 8
-    // (thread t owns chunk t % CPR; threads past the last whole group of CPR kept zeros)
-#pragma unroll
-    for (int q = tid; q < CPR * 32; q += NTH) {
-        const int c = q >> 5, v = q & 31;
-        const int col = col0 + c * 8 + (v & 7);
-        if ((v >> 4) >= nslot || col >= a.N) continue;
-        float t = 0.f;
-#pragma unroll
-        for (int j = 0; j < NTH / CPR; ++j) t += red[v * NTH + ((c + j * CPR) ^ v)];
-        atomicAdd(&a.stats[((int64_t)(b0 + (v >> 4)) * a.N + col) * 2 + ((v >> 3) & 1)], (double)t);
-    }
 }
 
 // Sum split-K partials and apply the epilogue.  Vector path: 8 output columns
@@ -249,12 +196,6 @@ __global__ void splitk_reduce_kernel(GemmArgs a) {
     else reduce_rows<1, false>(a, m, 1u, nout, o);
 }
 
-// 8 consecutive fp32 values from 16-byte-aligned LDS
-__device__ __forceinline__ void ld8(const float* p, float (&v)[8]) {
-    const float4 x = *(const float4*)p, y = *(const float4*)(p + 4);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w; v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
-}
-
 // Main loop: NS-stage LDS ring fed by global_load_lds_dwordx4 (direct to LDS, no
 // register staging), NS-1 K tiles in flight while one is consumed, one s_barrier
 // per K tile.  LDS rows are BK halves (64 or 128 bytes) with the 16-byte chunk
@@ -302,16 +243,11 @@ void gemm_kernel(GemmArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wn = wave / WM;
 
-    // XCD-aware block order: consecutive hardware block ids go round-robin over the
-    // 8 XCDs; give each XCD a contiguous range of logical tiles (XCD x: the nblk / 8
-    // tiles, one more for the first nblk % 8 XCDs, after those of XCDs < x), so that
-    // neighbouring tiles share that XCD's L2.  Neighbours share A rows (M-major order)
-    // or, when the weights are the larger operand, W columns (N-major order).
+    // XCD-aware block order.  Neighbours share A rows (M-major order) or, when the weights
+    // are the larger operand, W columns (N-major order).
     const int tiles_n = (a.N + NT - 1) / NT;
     const int tiles_m = (a.M + MT - 1) / MT;
-    const int nblk = tiles_m * tiles_n;
-    const int xcd = blockIdx.x & 7, per = nblk >> 3, extra = nblk & 7;
-    const int bid = xcd * per + min(xcd, extra) + (blockIdx.x >> 3);
+    const int bid = xcd_block(tiles_m * tiles_n);
     int tm, tn;
     if (a.n_major) {
         tn = bid / tiles_m;
@@ -321,11 +257,6 @@ void gemm_kernel(GemmArgs a) {
         tn = bid - tm * tiles_n;
     }
     const int m0 = tm * MT, n0 = tn * NT;
-    // sub-pixel conv (GemmArgs::subpix): the tile's phase (a tile never straddles two)
-    // and the first GEMM row of that phase
-    const bool subpix = AM == A_CONV3 && a.subpix;
-    const int sp_rows = a.M >> 2;
-    const int sp_ph = subpix ? m0 / sp_rows : 0, sp_base = sp_ph * sp_rows;
 
     const int kbeg = blockIdx.z * a.k_per_split;
     const int kend = min(a.K, kbeg + a.k_per_split);
@@ -349,20 +280,19 @@ void gemm_kernel(GemmArgs a) {
     const f16* zero = (const f16*)g_zero_page;
     constexpr uint32_t kOOB = 0x80000000u;
     const __amdgpu_buffer_rsrc_t rsB =
-        __builtin_amdgcn_make_buffer_rsrc((void*)a.Wt, (short)0, (subpix ? 4 : 1) * a.N * a.K * 2, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void*)a.Wt, (short)0, a.N * a.K * 2, 0x00020000);
     uint32_t voB[BI];
     int b_c[BI];
 #pragma unroll
     for (int i = 0; i < BI; ++i) {
         const int row = (i * NW + wave) * RPI + lr;
         b_c[i] = (pchunk ^ lds_swizzle<BKT>(row)) * 8;
-        voB[i] = (uint32_t)(((sp_ph * a.N + min(n0 + row, a.N - 1)) * a.K + b_c[i]) * 2);
+        voB[i] = (uint32_t)((min(n0 + row, a.N - 1) * a.K + b_c[i]) * 2);
     }
     int a_c[AI];          // element offset of the lane's chunk within the K tile
     int a_m[AI];          // dense: row (clamped)
     uint32_t voA[AI];     // dense: byte offset of (row, chunk) in A
-    uint32_t voA2[AI];    // byte offset of (row, chunk) in A2 (dense second source, conv tail)
-    uint32_t voA3[AI];    // conv: byte offset of (row, chunk) in A3
+    uint32_t voA2[AI];    // dense: byte offset of (row, chunk) in the second source A2
     int a_off[AI];        // conv: element offset of tap (0,0) of the lane's output pixel (+chunk)
     int a_vm[AI];         // conv: bit ky*3+kx set when that tap is inside the image
     int a_b[AI], a_oy[AI], a_ox[AI];  // conv geometry for the per-lane path
@@ -376,25 +306,6 @@ void gemm_kernel(GemmArgs a) {
             voA[i] = (uint32_t)((m * a.lda + a_c[i]) * 2);
             voA2[i] = a.A2 ? (uint32_t)((m * a.lda2 + a_c[i]) * 2) : 0u;
         } else {
-            voA2[i] = a.A2 ? (uint32_t)((m * a.lda2 + a_c[i]) * 2) : 0u;
-            voA3[i] = a.A3 ? (uint32_t)((m * a.lda3 + a_c[i]) * 2) : 0u;
-            if (subpix) {
-                // input pixel (iy, ix) of phase (py, px): 2x2 taps at rows iy + py - 1 + ty,
-                // columns ix + px - 1 + tx
-                const int hwi = a.Hin * a.Win, q = m - sp_base;
-                const int bb = q / hwi, r = q - bb * hwi, iy = r / a.Win, ix = r - iy * a.Win;
-                const int y0 = iy + (sp_ph >> 1) - 1, x0 = ix + (sp_ph & 1) - 1;
-                a_b[i] = bb; a_oy[i] = iy; a_ox[i] = ix;
-                a_off[i] = ((bb * a.Hin + y0) * a.Win + x0) * a.Cin + a_c[i];
-                int vm = 0;
-#pragma unroll
-                for (int ty = 0; ty < 2; ++ty)
-#pragma unroll
-                    for (int tx = 0; tx < 2; ++tx)
-                        if (y0 + ty >= 0 && y0 + ty < a.Hin && x0 + tx >= 0 && x0 + tx < a.Win) vm |= 1 << (ty * 2 + tx);
-                a_vm[i] = vm;
-                continue;
-            }
             const int hw = a.Ho * a.Wo;
             const int bb = m / hw, p = m - bb * hw;
             const int oy = p / a.Wo, ox = p - oy * a.Wo;
@@ -418,8 +329,6 @@ void gemm_kernel(GemmArgs a) {
         DENSE ? a.M * a.lda * 2 : a.Bn * a.Hin * a.Win * a.Cin * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsA2 = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.A2 ? a.A2 : a.A), (short)0, a.A2 ? a.M * a.lda2 * 2 : 0, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsA3 = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(a.A3 ? a.A3 : a.A), (short)0, a.A3 ? a.M * a.lda3 * 2 : 0, 0x00020000);
     // conv fast path: each K tile lies inside one tap (Cin % BKT == 0) and the input
     // is not upsampled, so the tap offset is one scalar per tile.  The K tiles of the
     // conv part go channel-chunk-major: the 9 taps of one BKT-channel chunk back to back
@@ -428,11 +337,10 @@ void gemm_kernel(GemmArgs a) {
     // that chunk is still in L2, rather than after a sweep over all Cin channels.  A
     // split-K block takes a contiguous range of virtual tiles.
     const bool conv_fast = AM == A_CONV3 && a.Cin % BKT == 0 && !a.upsample;
-    const int ntap = subpix ? 4 : 9;  // 3x3 taps, or the sub-pixel form's 2x2
     int tap_next = 0, c_next = 0;  // tap / channel of the next tile issued (fast path)
     if (conv_fast) {
-        const int v0 = kbeg / BKT, chunk = v0 / ntap;
-        tap_next = v0 - chunk * ntap;
+        const int v0 = kbeg / BKT, chunk = v0 / 9;
+        tap_next = v0 - chunk * 9;
         c_next = chunk * BKT;
     }
 
@@ -466,21 +374,11 @@ void gemm_kernel(GemmArgs a) {
                     dma(k < kend ? src : zero, sA + (i * NW + wave) * RPI * BKT);
                 }
             }
-        } else if (a.A2 && k0 >= a.K1) {
-            // conv dense tail: whole tiles (K1, K2, K multiples of the K tile), after
-            // every conv tile, so the fast path's tap counters are not advanced
-            if (!a.A3 || k0 < a.K2) {
-#pragma unroll
-                for (int i = 0; i < AI; ++i) bdma(rsA2, voA2[i], (k0 - a.K1) * 2, sA + (i * NW + wave) * RPI * BKT);
-            } else {
-#pragma unroll
-                for (int i = 0; i < AI; ++i) bdma(rsA3, voA3[i], (k0 - a.K2) * 2, sA + (i * NW + wave) * RPI * BKT);
-            }
         } else if (conv_fast) {
-            const int tap = tap_next, ky = subpix ? tap >> 1 : tap / 3, kx = tap - ky * (subpix ? 2 : 3);
+            const int tap = tap_next, ky = tap / 3, kx = tap - ky * 3;
             const int toff = (ky * a.Win + kx) * a.Cin + c_next;
             kw = tap * a.Cin + c_next;
-            if (++tap_next == ntap) { tap_next = 0; c_next += BKT; }
+            if (++tap_next == 9) { tap_next = 0; c_next += BKT; }
 #pragma unroll
             for (int i = 0; i < AI; ++i) {
                 const bool ok = ((a_vm[i] >> tap) & 1) && !(tail && k0 + a_c[i] >= kend);
@@ -850,9 +748,8 @@ void gemm_kernel(GemmArgs a) {
     // per-channel output statistics (GroupNorm of the consumer): this thread's 8
     // columns over its rows, for the tile's first image (slot 0) and the next (slot 1)
     const bool do_st = a.stats != nullptr && !narrow;
-    // (sub-pixel conv: statistics rows counted within the phase, stats_hw = Hin * Win)
-    const int st_b0 = do_st ? (m0 - sp_base) / a.stats_hw : 0;
-    const int st_mb = sp_base + (st_b0 + 1) * a.stats_hw;  // first row of the next image
+    const int st_b0 = do_st ? m0 / a.stats_hw : 0;
+    const int st_mb = (st_b0 + 1) * a.stats_hw;  // first row of the next image
     float st[2][2][8];
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl)
@@ -955,13 +852,7 @@ void gemm_kernel(GemmArgs a) {
                 f16* oh = (f16*)&o;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) oh[e] = (f16)v[e];
-                int mo = m;  // output row (sub-pixel conv: the phase's pixel in the upsampled image)
-                if (subpix) {
-                    const int hwi = a.Hin * a.Win, q = m - sp_base;
-                    const int bb = q / hwi, r = q - bb * hwi, iy = r / a.Win, ix = r - iy * a.Win;
-                    mo = (bb * a.Ho + 2 * iy + (sp_ph >> 1)) * a.Wo + 2 * ix + (sp_ph & 1);
-                }
-                *(uint4*)((f16*)a.C + (int64_t)mo * a.ldc + nout) = o;
+                *(uint4*)((f16*)a.C + (int64_t)m * a.ldc + nout) = o;
                 if (do_rs) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
@@ -986,7 +877,10 @@ void gemm_kernel(GemmArgs a) {
             }
         }
     }
-    if (do_st) stats_flush<NTH, NT / 8>(a, st, st_b0, min(a.M, m0 + MT) - 1 - sp_base, n0, (float*)smem);
+    if (do_st) {
+        const int m_last = min(a.M, m0 + MT) - 1;
+        stats_flush<NTH, NT / 8>(a, st, st_b0, m_last / a.stats_hw != st_b0 ? 2 : 1, n0, (float*)smem);
+    }
     if (do_rs) {
         // the cpr threads of a row are consecutive lanes, each 8 of them one 64-column
         // group: add their partial sums; the first of the 8 stores the group's partial
@@ -1102,51 +996,69 @@ struct Cfg {
     double t_fix;         // per-block prologue + epilogue time
     int spr;              // split slots per modelled round of the summing block's tail
     double conv_f;        // rate factor with the implicit-conv A (the tap gather)
+    int patch;            // conv3_patch_kernel's tile shape, or -1
+    double t_round;       // the summing block's time per modelled round
 };
 // 0: 256x128, 8 waves of 64x64, BK 64, 2-stage ring (96 KB: one block per CU)
 // 1: 128x128, 8 waves of 64x32, BK 64, 2-stage ring (64 KB: two per CU, 4 waves per SIMD)
 // 2: 128x64,  8 waves of 32x32, BK 64, 3-stage ring (72 KB: two per CU, 4 waves per SIMD)
 // 3: 64x160,  4 waves of 32x80 (16x16x32 MFMAs), BK 64, 2-stage ring (56 KB: two per CU)
-// Rates and fixed costs from dense GEMMs that give every CU one or two blocks, at
-// K = 512 and 4096 (the difference gives the rate, the rest the fixed cost).  The
-// 128x128 two-block rate is set above that fit (3.54): the 64x64 convs over the up
-// path's concatenated inputs run two splits as co-resident pairs faster than it
-// predicts (640 -> 320: 56.6 us with 2 splits against 62.4 with 4), and whole forwards
-// compared in one call take 5.09 against 5.10 ms (B=2 64x64), 9.69 against 9.78 (96x96)
-// and 21.45 against 21.45 (B=16).  The implicit-conv A (a tap gather per row) costs the
-// 64-column tile about 20% of its rate.
-// The 64x160 tile covers N = 320 with no padded column and M = 8192 with 256 tiles, so it
-// fills the chip where 128-row tiles leave a quarter of the CUs idle, but its own rate is
-// lower (4 waves, 46 FLOP per operand byte against 64): its parameters are fitted to 18
-// UNet GEMMs timed with both tiles in one forward (B=2 and 16, 64x64 latents).  In whole
-// forwards the planner then takes it for the 64x64 level's convs at B=2 (M = 8192,
-// N = 320: 38.5 against 41.8 us at K = 2880, 83.4 against 93.0 at K = 8640), the 77-token
-// cross K/V GEMM (21.2 against 24.6 us) and two B=16 feed-forward outputs, each faster
-// than before; it loses at larger M (B=16 conv, M = 65536: 192.6 against 178.3 us).
-constexpr int kNumCfg = 4;
-// The tail model counts one slot per round for the 128-row tiles and two for the others
-// (their kernels load 1, 2, 4 and 2 slots per round): moving the 128x128 tile to its
-// kernel's 2 sends the 64x64 and 48x48 levels' concat convs from the reduce launch to the
-// in-kernel sum and changed them by -10% to +15% each, no gain over a forward.
-const Cfg kCfgs[kNumCfg] = {{256, 128, 1, 3.5e12, 3.5e12, 4.5e-6, 1, 1.0},
-                            {128, 128, 2, 2.76e12, 3.9e12, 3.0e-6, 1, 1.0},
-                            {128, 64, 2, 2.23e12, 3.03e12, 2.5e-6, 2, 0.8},
-                            {64, 160, 2, 2.0e12, 3.4e12, 6.0e-6, 2, 0.9}};
+// 4 ..: the patch-resident conv kernel's shapes (k_conv.hip): 16x16 pixels x 128 or 160
+// channels (8 waves, one block per CU), two 8x8 sub-tiles x 80 or 64 channels (4 waves, two)
+// Rates and fixed costs of 0..3 from dense GEMMs that give every CU one or two blocks, at
+// K = 512 and 4096 (the difference gives the rate, the rest the fixed cost).  The 64x160
+// tile covers N = 320 with no padded column and M = 8192 with 256 tiles, so it fills the
+// chip where 128-row tiles leave a quarter of the CUs idle, but its own rate is lower (4
+// waves, 46 FLOP per operand byte against 64).  The implicit-conv A (a tap gather per row)
+// costs the 64-column tile about 20% of its rate.
+// 4 ..: fitted to 1700 launches over 44 conv shapes (8x8 to 512x512 pixels, 64 to 2560
+// channels, batches 1 to 16, ragged sizes; every shape and split count timed): the planner's
+// choice is within 3% of the best of them on all but two (4%), and always a shape of
+// this kernel, so the convs it can take are planned among these alone.
+constexpr int kNumGemm = 4, kNumCfg = kNumGemm + kNumPatch;
+const Cfg kCfgs[kNumCfg] = {{256, 128, 1, 3.5e12, 3.5e12, 4.5e-6, 1, 1.0, -1, 0.9e-6},
+                            {128, 128, 2, 2.76e12, 3.9e12, 3.0e-6, 1, 1.0, -1, 0.9e-6},
+                            {128, 64, 2, 2.23e12, 3.03e12, 2.5e-6, 2, 0.8, -1, 0.9e-6},
+                            {64, 160, 2, 2.0e12, 3.4e12, 6.0e-6, 2, 0.9, -1, 0.9e-6},
+                            {256, 128, 1, 6.8e12, 6.8e12, 8.2e-6, 1, 1.0, 0, 1.0e-6},
+                            {256, 160, 1, 6.0e12, 6.0e12, 8.8e-6, 1, 1.0, 1, 1.2e-6},
+                            {128, 80, 2, 5.07e12, 5.2e12, 4.75e-6, 1, 1.0, 2, 0.39e-6},
+                            {128, 64, 2, 4.63e12, 5.08e12, 4.0e-6, 1, 1.0, 3, 0.33e-6}};
 // full kernel names, as the instantiations (tile configuration, A mode: 0 dense, 1 implicit conv,
 // then the MFMA)
-const char* const kNames[kNumCfg][2] = {{"gemm_kernel<256,128,4,2,64,2,0,32>", "gemm_kernel<256,128,4,2,64,2,1,32>"},
+const char* const kNames[kNumGemm][2] = {{"gemm_kernel<256,128,4,2,64,2,0,32>", "gemm_kernel<256,128,4,2,64,2,1,32>"},
                                         {"gemm_kernel<128,128,2,4,64,2,0,32>", "gemm_kernel<128,128,2,4,64,2,1,32>"},
                                         {"gemm_kernel<128,64,4,2,64,3,0,32>", "gemm_kernel<128,64,4,2,64,3,1,32>"},
                                         {"gemm_kernel<64,160,2,2,64,2,0,16>", "gemm_kernel<64,160,2,2,64,2,1,16>"}};
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// In-kernel split-K sum: tile counters at the head of the workspace (one per tile),
-// the slots the summing block loads per round (as the kernel's SPR), and the
-// modelled cost of its tail.
+// In-kernel split-K sum: tile counters at the head of the workspace (one per tile).
 constexpr int kMaxSplitTiles = 16384;
 constexpr size_t kCounterBytes = kMaxSplitTiles * sizeof(unsigned);
-constexpr double kFixBase = 1.0e-6, kFixRound = 0.9e-6;
+// Split costs outside the kernels' own time, for gemm_kernel and conv3_patch_kernel: the fp32
+// partial round trip's rate (mostly L2 / Infinity Cache resident), the in-kernel sum's fixed
+// part, the reduce launch.
+struct SplitCost {
+    double rate, fix, red;
+};
+constexpr SplitCost kSplit[2] = {{20.0e12, 1.0e-6, 5.5e-6}, {38.0e12, 2.9e-6, 4.2e-6}};
+
+const char* cfg_name(int ci, const GemmArgs& a) {
+    return ci < kNumGemm ? kNames[ci][a.amode == A_CONV3] : conv_patch_name(kCfgs[ci].patch, a.subpix);
+}
+
+int cfg_tiles(int ci, const GemmArgs& a) {
+    const int tm = ci < kNumGemm ? ceil_div(a.M, kCfgs[ci].mt) : conv_patch_tiles_m(kCfgs[ci].patch, a);
+    return tm * ceil_div(a.N, kCfgs[ci].nt);
+}
+
+// The convs the patch-resident kernel takes.  (Pixel indices stay below 2^24: 64 channels of
+// each fit the 2 GiB an operand may have.)
+bool patch_ok(const GemmArgs& a) {
+    return a.amode == A_CONV3 && a.stride == 1 && !a.upsample && a.Cin % 64 == 0 && a.N % 8 == 0 &&
+           a.out_mode != OUT_F32_NCHW && !a.geglu && !a.row_part && !a.ln_part;
+}
 
 // The epilogue keeps output statistics for two images per tile: the MT rows of a tile
 // (MT-aligned) must not reach a third image.
@@ -1156,50 +1068,55 @@ bool stats_tile_ok(int mt, int hw) { return hw >= mt || mt == 2 * hw; }
 // spread evenly over the 256 CUs; the busiest CU runs its blocks two at a time where
 // the tile allows two per CU (a lone block cannot keep a CU busy: rate1 < rate2),
 // each round paying a fixed prologue / epilogue cost.  A split K adds the fp32
-// partial round trip (mostly L2 / Infinity Cache resident) and the serial tail of
-// the block that sums a tile's partials.
+// partial round trip and the serial tail of the block that sums a tile's partials, or
+// the reduce launch.
 void plan(const GemmArgs& a, int& ci, int& splits, int& kps, bool& fix) {
-    const int nkt = ceil_div(a.K, 64);
+    const bool patch = patch_ok(a);
+    const int nkt = ceil_div(a.K, 64), nc = patch ? a.Cin / 64 : 0, ntap = a.subpix ? 4 : 9;
     double best = 1e30;
-    ci = 1; splits = 1; kps = nkt * 64; fix = false;
-    for (int c = 0; c < kNumCfg; ++c) {
+    ci = patch ? kNumGemm : 1; splits = 1; kps = nkt * 64; fix = false;
+    for (int c = patch ? kNumGemm : 0; c < (patch ? kNumCfg : kNumGemm); ++c) {
         const Cfg& g = kCfgs[c];
-        if (a.geglu && g.nt % 128) continue;  // GEGLU pairs 32-column blocks within a 64-wide wave tile
-        // LayerNorm row partials: one per 64 columns, summed by 8 consecutive lanes
-        if (a.row_part && g.nt % 64) continue;
-        // the LayerNorm consumer's epilogue runs 5-8% slower in the 4-wave 64x160 tile than
-        // the 128x128 tile at K = 1280 (M = 1152, N = 3840: 27.8 against 25.7 us), which
-        // the model does not see
-        if (a.ln_part && g.mt == 64) continue;
-        // (sub-pixel conv: whole phases per tile; statistics images of Hin * Win rows)
-        if (a.subpix && (a.M >> 2) % g.mt) continue;
-        if (a.stats && !stats_tile_ok(g.mt, a.subpix ? a.Hin * a.Win : a.stats_hw)) continue;
-        const int tiles = ceil_div(a.M, g.mt) * ceil_div(a.N, g.nt);
+        if (patch) {
+            if (a.subpix && !conv_patch_subpix(g.patch)) continue;
+        } else {
+            if (a.geglu && g.nt % 128) continue;  // GEGLU pairs 32-column blocks within a 64-wide wave tile
+            // LayerNorm row partials: one per 64 columns, summed by 8 consecutive lanes
+            if (a.row_part && g.nt % 64) continue;
+            // the LayerNorm consumer's epilogue runs 5-8% slower in the 4-wave 64x160 tile than
+            // the 128x128 tile at K = 1280 (M = 1152, N = 3840: 27.8 against 25.7 us), which
+            // the model does not see
+            if (a.ln_part && g.mt == 64) continue;
+            if (a.stats && !stats_tile_ok(g.mt, a.stats_hw)) continue;
+        }
+        const int tiles = cfg_tiles(c, a);
+        const SplitCost& sc = kSplit[patch];
         static const int cand[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
         for (int s : cand) {
             if (s > 1 && nkt / s < 4) break;
-            const int kt_per = ceil_div(nkt, s);
-            const int se = ceil_div(nkt, kt_per);
+            // (a patch block takes whole chunks of ntap steps, see the kernel's K order)
+            int kt_per = ceil_div(nkt, s), se = ceil_div(nkt, kt_per);
+            if (patch) {
+                if (nc * ntap == nkt) kt_per = ntap * ceil_div(nc, s);
+                se = s;
+                if (s > nc + nkt - nc * ntap) break;
+            }
             const long blocks = (long)tiles * se;
             const long load = (blocks + 255) / 256;  // blocks on the busiest CU
             const double w = 2.0 * g.mt * g.nt * kt_per * 64.0;
             const long pairs = g.per_cu >= 2 ? load / 2 : 0, singles = load - 2 * pairs;
             const double cf = a.amode == A_CONV3 ? g.conv_f : 1.0;
             double t = pairs * (2.0 * w / (g.rate2 * cf) + g.t_fix) + singles * (w / (g.rate1 * cf) + g.t_fix);
-            // a split adds the partial round trip, and either the reduce launch (about
-            // 5.5 us, 2 us more with statistics) or the serial tail of each tile's last
-            // block (the count, then its rounds of slot loads)
             bool fx = false;
             if (se > 1) {
-                const double part = (double)se * a.M * a.N * 8.0 / 20.0e12;
+                const double part = (double)se * a.M * a.N * 8.0 / sc.rate;
                 // (with output statistics only the in-kernel sum: the reduce keeps none)
-                const double t_red = (a.stats || a.row_part || a.ln_part || a.subpix) ? 1e30 : part + 5.5e-6;
-                const int rounds = ceil_div(se, g.spr);
-                const double t_fix = tiles <= kMaxSplitTiles ? part + kFixBase + kFixRound * rounds : 1e30;
+                const double t_red = (a.stats || a.row_part || a.ln_part || a.subpix) ? 1e30 : part + sc.red;
+                const double t_fix = tiles <= kMaxSplitTiles ? part + sc.fix + g.t_round * ceil_div(se, g.spr) : 1e30;
                 fx = t_fix < t_red;
                 t += fx ? t_fix : t_red;
             }
-            if (t < best * 0.98) { best = t; ci = c; splits = se; kps = kt_per * 64; fix = fx; }
+            if (t < best * (patch ? 0.999 : 0.98)) { best = t; ci = c; splits = se; kps = kt_per * 64; fix = fx; }
         }
     }
 }
@@ -1212,7 +1129,7 @@ const char* gemm_kernel_name(const GemmArgs& a) {
     int ci, splits, kps;
     bool fix;
     plan(a, ci, splits, kps, fix);
-    return kNames[ci][a.amode == A_CONV3];
+    return cfg_name(ci, a);
 }
 
 size_t gemm_counter_bytes() { return kCounterBytes; }
@@ -1224,7 +1141,7 @@ size_t gemm_workspace_bytes(const GemmArgs& a) {
     plan(a, ci, splits, kps, fix);
     if (splits == 1) return 0;
     const Cfg& g = kCfgs[ci];
-    const size_t tiles = (size_t)ceil_div(a.M, g.mt) * ceil_div(a.N, g.nt);
+    const size_t tiles = cfg_tiles(ci, a);
     return kCounterBytes + (fix ? tiles * g.mt * g.nt : (size_t)a.M * a.N) * splits * sizeof(float);
 }
 
@@ -1261,7 +1178,10 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
     plan(a, ci, splits, kps, fix);
     if (a.A2 == nullptr) a.K1 = a.K;
     if (a.A3 == nullptr) a.K2 = a.K;
-    if (a.A3 && (a.amode != A_CONV3 || !a.A2)) return hipErrorInvalidValue;
+    const Cfg& g = kCfgs[ci];
+    // a conv's dense tail and the sub-pixel form are the patch kernel's
+    if ((a.A3 && (a.amode != A_CONV3 || !a.A2)) || ((a.subpix || (a.amode == A_CONV3 && a.A2)) && g.patch < 0))
+        return hipErrorInvalidValue;
     // (a consumer thread sums up to 10 row partials; 2 or 4 threads per tile row)
     if (a.ln_part && (a.amode != A_DENSE || a.A2 || !a.ln_colsum || a.out_mode != OUT_F16 || (a.N & 7) ||
                       (a.K & 63) || a.K > 1280 || !(a.ln_eps > 0.f) || (splits > 1 && !fix)))
@@ -1269,17 +1189,15 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
     if (a.row_part && (a.out_mode != OUT_F16 || a.geglu || (a.N & 63) || (splits > 1 && !fix)))
         return hipErrorInvalidValue;
     if (a.subpix) {
-        if (a.amode != A_CONV3 || a.upsample || a.stride != 1 || a.A2 || a.A3 || a.Cin % 64 || a.K != 4 * a.Cin ||
-            a.Ho != 2 * a.Hin || a.Wo != 2 * a.Win || a.M != a.Bn * a.Ho * a.Wo || a.res || a.row_part ||
-            a.ln_part || a.geglu || a.out_mode != OUT_F16 || (a.N & 7) || (a.M >> 2) % kCfgs[ci].mt ||
-            (splits > 1 && !fix) || (a.stats && a.stats_hw != a.Ho * a.Wo))
+        if (a.A2 || a.K != 4 * a.Cin || a.Ho != 2 * a.Hin || a.Wo != 2 * a.Win || a.M != a.Bn * a.Ho * a.Wo || a.res ||
+            a.out_mode != OUT_F16 || (splits > 1 && !fix))
             return hipErrorInvalidValue;
-        if (a.stats) a.stats_hw = a.Hin * a.Win;  // the kernel counts rows within a phase
+    } else if (g.patch >= 0) {
+        if (a.K1 != 9 * a.Cin || a.Ho != a.Hin || a.Wo != a.Win || a.M != a.Bn * a.Ho * a.Wo) return hipErrorInvalidValue;
     }
     if (a.amode == A_CONV3 && a.A2 &&
-        (a.K1 != 9 * a.Cin || a.K1 % 64 || a.K2 % 64 || a.K % 64 || a.K2 <= a.K1 || a.K <= a.K1 ||
-         (a.A3 && a.K2 >= a.K) || a.stride != 1 || a.upsample || a.Ho != a.Hin || a.Wo != a.Win ||
-         a.M != a.Bn * a.Ho * a.Wo || a.lda2 < a.K2 - a.K1 || (a.A3 && a.lda3 < a.K - a.K2)))
+        (a.K2 % 64 || a.K % 64 || a.K2 <= a.K1 || (a.A3 && a.K2 >= a.K) || a.lda2 < a.K2 - a.K1 ||
+         (a.A3 && a.lda3 < a.K - a.K2)))
         return hipErrorInvalidValue;
     a.splits = splits;
     a.k_per_split = kps;
@@ -1303,11 +1221,10 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
     if (a.amode == A_CONV3 && (2 * (int64_t)a.Bn * a.Hin * a.Win * a.Cin > lim ||
                                (a.A2 && 2 * (int64_t)a.M * a.lda2 > lim) || (a.A3 && 2 * (int64_t)a.M * a.lda3 > lim)))
         return hipErrorInvalidValue;
-    const Cfg& g = kCfgs[ci];
     if (a.stats && (a.out_mode != OUT_F16 || a.geglu || (a.N & 7) || a.stats_hw < 64 ||
-                    !stats_tile_ok(g.mt, a.stats_hw)))
+                    (g.patch < 0 ? !stats_tile_ok(g.mt, a.stats_hw) : a.stats_hw != a.Ho * a.Wo)))
         return hipErrorInvalidValue;
-    dim3 grid(ceil_div(a.M, g.mt) * ceil_div(a.N, g.nt), 1, splits);
+    const dim3 grid(cfg_tiles(ci, a), 1, splits);
     // algorithmic traffic: A once (the conv source image, not its im2col), W once, output
     // (+ residual) once.  A split's fp32 partials are overhead, not algorithmic traffic:
     // they are counted nowhere, and the reduce launch reports no algorithmic bytes
@@ -1321,8 +1238,9 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
     const double kop = a.subpix ? 9.0 * a.Cin : (double)a.K;
     const double flops = 2.0 * a.M * a.N * kop;
     const double k_bytes = a_bytes + 2.0 * a.N * kop + out_bytes;
-    launch_timed(kNames[ci][a.amode == A_CONV3], flops, k_bytes, [&] {
-        if (a.amode == A_DENSE) launch_cfg<A_DENSE>(ci, grid, a, s);
+    launch_timed(cfg_name(ci, a), flops, k_bytes, [&] {
+        if (g.patch >= 0) conv_patch_launch(g.patch, a, s);
+        else if (a.amode == A_DENSE) launch_cfg<A_DENSE>(ci, grid, a, s);
         else launch_cfg<A_CONV3>(ci, grid, a, s);
     });
     hipError_t e = hipGetLastError();

@@ -161,6 +161,14 @@ const char* gemm_kernel_name(const GemmArgs& a);  // tile variant the launch wil
 hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s);
 // Sum a.splits fp32 partials [splits][M][N] at a.partial and run the epilogue.
 hipError_t splitk_reduce_launch(const GemmArgs& a, double bytes, hipStream_t s);
+// The patch-resident 3x3 conv kernel (k_conv.hip): tile shape `cfg` of kNumPatch, for the
+// A_CONV3 GEMMs that gemm_launch sends there (stride 1, no upsample, Cin % 64 == 0, N % 8 ==
+// 0, fp16 or fp32 rows out, any splits).
+constexpr int kNumPatch = 4;
+int conv_patch_tiles_m(int cfg, const GemmArgs& a);
+bool conv_patch_subpix(int cfg);  // the shape has a sub-pixel form
+const char* conv_patch_name(int cfg, bool subpix);
+void conv_patch_launch(int cfg, const GemmArgs& a, hipStream_t s);
 // Sub-pixel weights of a 3x3 conv that follows a 2x nearest upsampling (GemmArgs::subpix):
 // w3 [Cout][3][3][Cin] -> w4 [4 phases][Cout][2][2][Cin], phase = 2 py + px.  Tap (ty, tx)
 // of phase (py, px) is the fp32 sum of the 3x3 taps (ky, kx) with ty = (py + ky + 1) / 2 - py

@@ -305,6 +305,24 @@ def test_conv2d(op_engine, B, H, W, Ci, Co, k, stride, ups, temb, res):
     assert np.abs(got - ref).max() < 3e-2
 
 
+@pytest.mark.parametrize("B,H,W,Ci,Co,temb,res", [
+    (1, 8, 8, 64, 8, False, False),        # one sub-tile of the two-sub-tile block, one chunk, N < 16
+    (3, 8, 8, 128, 72, True, True),        # odd sub-tile count, last column tile of 8
+    (1, 9, 17, 64, 168, False, True),      # one pixel past a sub-tile in both directions
+    (2, 7, 15, 192, 88, True, False),      # one pixel short
+    (1, 48, 47, 128, 128, False, True),    # a ragged column of sub-tiles
+    (1, 256, 256, 64, 136, False, False),  # 16x16 sub-tiles, last column tile of 8
+    (5, 64, 64, 320, 320, True, True),     # 160-column tiles
+    (1, 250, 243, 128, 128, True, False),  # 16x16 sub-tiles, both directions ragged
+    (2, 8, 8, 1280, 1280, False, True),    # split K with the reduce launch
+    (1, 16, 16, 704, 320, True, False),    # 11 chunks over uneven splits
+])
+def test_conv_patch_tiles(op_engine, B, H, W, Ci, Co, temb, res):
+    """Edges of the patch-resident 3x3 kernel's tiles: 8x8 and 16x16 sub-tiles of ragged
+    images, column tiles of 64, 80, 128 and 160, split K at chunk boundaries."""
+    test_conv2d(op_engine, B, H, W, Ci, Co, 3, 1, False, temb, res)
+
+
 @pytest.mark.parametrize("M,N,K", [
     (8192, 320, 320),    # the attention output projection's shape (residual loaded up front)
     (128, 1280, 5120),   # split K
