@@ -18,6 +18,9 @@ __device__ __forceinline__ void wait_vmcnt_lgkm0() {
     __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0x0 << 8) | ((N >> 4) << 14));
 }
 
+// lgkmcnt(0) alone
+__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xF | (0x7 << 4) | (0x0 << 8) | (0x3 << 14)); }
+
 // Sum the per-thread column statistics of a block over the threads that own the same
 // 8 columns (thread t owns chunk t % CPR; chunk c covers columns col0 + 8c ..) through
 // LDS and add them to the per-(image, channel) fp64 statistics of images b0 and (nslot 2)
@@ -66,9 +69,10 @@ __device__ __forceinline__ void ld8(const float* p, float (&v)[8]) {
 // Logical block id of this workgroup: hardware ids go round-robin over the 8 XCDs; each XCD
 // gets a contiguous range of the nblk logical tiles (XCD x: nblk / 8 tiles, one more for the
 // first nblk % 8 XCDs), so that neighbouring tiles share that XCD's L2.
-__device__ __forceinline__ int xcd_block(int nblk) {
-    const int xcd = blockIdx.x & 7, per = nblk >> 3, extra = nblk & 7;
-    return xcd * per + min(xcd, extra) + (blockIdx.x >> 3);
+// (vb: the hardware id, or a persistent block's id plus a multiple of its grid.)
+__device__ __forceinline__ int xcd_block(int nblk, int vb) {
+    const int xcd = vb & 7, per = nblk >> 3, extra = nblk & 7;
+    return xcd * per + min(xcd, extra) + (vb >> 3);
 }
 
 }  // namespace sdu

@@ -92,7 +92,7 @@ void conv3_patch_kernel(GemmArgs a) {
     const int nbx = (a.Win + TW - 1) / TW, nby = (a.Hin + TW - 1) / TW, spi = nbx * nby, nsub = a.Bn * spi;
     const int tpp = (nsub + NSUB - 1) / NSUB;  // tiles (per phase)
     const int tiles_m = NTAP == 4 ? 4 * tpp : tpp, tiles_n = (a.N + NT - 1) / NT;
-    const int bid = xcd_block(tiles_m * tiles_n);
+    const int bid = xcd_block(tiles_m * tiles_n, blockIdx.x);
     int tm, tn;
     if (a.n_major) {
         tn = bid / tiles_m;
@@ -515,9 +515,9 @@ void conv_patch_launch(int cfg, const GemmArgs& a, hipStream_t s) {
         case 1: SDU_LAUNCH((conv3_patch_kernel<16, 1, 128, 4, 2, 4, 4, 2>), grid, blk, 0, s, a); break;
         case 2: SDU_LAUNCH((conv3_patch_kernel<16, 1, 160, 4, 2, 9, 3, 2>), grid, blk, 0, s, a); break;
         case 4: SDU_LAUNCH((conv3_patch_kernel<8, 2, 80, 4, 1, 9, 3, 2>), grid, blk, 0, s, a); break;
-        case 5: SDU_LAUNCH((conv3_patch_kernel<8, 2, 80, 4, 1, 4, 2, 2>), grid, blk, 0, s, a); break;
+        case 5: SDU_LAUNCH((conv3_patch_kernel<8, 2, 80, 4, 1, 4, 4, 1>), grid, blk, 0, s, a); break;
         case 6: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 9, 3, 2>), grid, blk, 0, s, a); break;
-        case 7: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 4, 2, 2>), grid, blk, 0, s, a); break;
+        case 7: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 4, 4, 1>), grid, blk, 0, s, a); break;
     }
 }
 

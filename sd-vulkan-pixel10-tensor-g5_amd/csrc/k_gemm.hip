@@ -4,18 +4,16 @@
 // v_mfma_f32_32x32x16_f16.  Replaces the reference's matmul_f32.comp (MM) and
 // every conv route of vk_engine.cpp:578-608 (1x1 GEMM, Winograd, im2col + GEMM):
 //   * A_DENSE: A is row-major [M, lda]; columns [K1, K) may come from a second
-//     source (the 1x1 shortcut over the up-path concat, vk_engine.cpp:634, :754).
+//     source.  K (or the split point) a multiple of 64 and N of 8, which every product of
+//     the networks has, goes to gemm_dense_kernel (k_dense.hip) instead, except ReLU and
+//     the odd epilogue combinations (dense_ok).
 //   * A_CONV3: A is the implicit im2col of an NHWC image for a 3x3 conv, pad 1, for the
 //     convs the patch-resident kernel (k_conv.hip) does not take: stride 2 (downsample,
 //     :689-692), nearest-2x upsample folded into the index math (upsample, :693-697), or
 //     channel counts outside its multiples.  K index = tap*Cin + ci.
 // Epilogue (fused; the reference runs these as separate AB/AB2/ADD/GEGLU passes):
 // + bias[n] + bias2[n] (fp32 time projection), GEGLU over interleaved a/b column
-// blocks, + residual, activation (ReLU / quick-GELU), store fp16 / fp32 / fp32-NCHW.  A LayerNorm (layernorm_f32.comp,
-// vk_engine.cpp:652, :658, :666) between two GEMMs runs inside them: the producer adds
-// each output row's sum and sum of squares into a row-statistics buffer, and the
-// consumer, reading the un-normalised rows as A, applies rstd * (acc - mean * colsum(W))
-// with the LayerNorm's affine folded into its W and bias.
+// blocks, + residual, activation (ReLU / quick-GELU), store fp16 / fp32 / fp32-NCHW.
 // Split-K, two ways: the last block of a tile to arrive sums the tile's fp32 partials
 // and runs the epilogue (few splits), or a reduce kernel does (many splits).
 #include "gemm_common.h"
@@ -247,7 +245,7 @@ void gemm_kernel(GemmArgs a) {
     // are the larger operand, W columns (N-major order).
     const int tiles_n = (a.N + NT - 1) / NT;
     const int tiles_m = (a.M + MT - 1) / MT;
-    const int bid = xcd_block(tiles_m * tiles_n);
+    const int bid = xcd_block(tiles_m * tiles_n, blockIdx.x);
     int tm, tn;
     if (a.n_major) {
         tn = bid / tiles_m;
@@ -454,34 +452,12 @@ void gemm_kernel(GemmArgs a) {
     for (int i = 0; i < (MF == 16 ? FM16 : 1); ++i)
 #pragma unroll
         for (int j = 0; j < (MF == 16 ? FN16 : 1); ++j) acc16[i][j] = floatx4{};
-    // LayerNorm consumer: the PPT consecutive lanes of tile row t / PPT load its 64-column
-    // partials j = t % PPT, + PPT, ... (issued before the first K tiles, added after),
-    // and thread t < NT the column sum of tile column t
-    constexpr int PPT = NTH / MT, MAXP = 20 / PPT;  // lanes per row, partials per lane (K <= 1280)
-    const bool lnc = DENSE && a.ln_part != nullptr;
-    float2 ln_v[MAXP];
-    float ln_cs_t = 0.f;
-    if (lnc) {
-        const int mm = min(m0 + tid / PPT, a.M - 1), T = a.K >> 6;
-#pragma unroll
-        for (int i = 0; i < MAXP; ++i) {
-            const int j = tid % PPT + i * PPT;
-            ln_v[i] = j < T ? *(const float2*)(a.ln_part + ((int64_t)j * a.M + mm) * 2) : make_float2(0.f, 0.f);
-        }
-        if (tid < NT && n0 + tid < a.N) ln_cs_t = a.ln_colsum[n0 + tid];
-    }
-
     // fragment addressing: row (base + lrow), logical chunk 2*ks + (lane>>5);
     // every fragment base row is a multiple of 32, so the swizzle depends on lrow only
     const int lrow = lane & 31, hl = lane >> 5, sw = lds_swizzle<BKT>(lrow);
 #pragma unroll
     for (int p = 0; p < NS - 1; ++p)
         if (p < nk) issue(p, p);
-    float ln_s1 = 0.f, ln_s2 = 0.f;
-    if (lnc) {
-#pragma unroll
-        for (int i = 0; i < MAXP; ++i) { ln_s1 += ln_v[i].x; ln_s2 += ln_v[i].y; }
-    }
     for (int kt = 0; kt < nk; ++kt) {
         // tile kt must have landed; the tiles issued after it may still be in flight
         wait_tiles<LPT, NS - 2>(min(NS - 2, nk - 1 - kt));
@@ -566,20 +542,6 @@ void gemm_kernel(GemmArgs a) {
 
     // ---- epilogue
     const int col_l = lane & 31, rq = (lane >> 5) * 4;
-    float2 ln_rs = make_float2(1.f, 0.f);  // (rstd, -mean * rstd) of row tid / PPT
-    if (lnc) {
-        // the row's PPT lanes add their partials
-#pragma unroll
-        for (int off = 1; off < PPT; off <<= 1) {
-            ln_s1 += __shfl_xor(ln_s1, off);
-            ln_s2 += __shfl_xor(ln_s2, off);
-        }
-        // one-pass statistics as the reference's layernorm_f32.comp (clamped at 0)
-        const float inv_k = 1.0f / (float)a.K;
-        const float mean = ln_s1 * inv_k;
-        const float rstd = rsqrtf(fmaxf(ln_s2 * inv_k - mean * mean, 0.f) + a.ln_eps);
-        ln_rs = make_float2(rstd, -mean * rstd);
-    }
     if (a.partial && !a.fixup) {
         // split K, reduce kernel: fp32 partial [split][M][N]
         float* P = a.partial + (int64_t)blockIdx.z * a.M * a.N;
@@ -714,12 +676,6 @@ void gemm_kernel(GemmArgs a) {
     static_assert(PR * CST * 4 <= NS * STAGE * 2, "C pass fits the operand LDS");
     static_assert(NTH * 32 * 4 <= NS * STAGE * 2, "statistics flush fits the operand LDS");
     float* Cs = (float*)smem;
-    // LayerNorm consumer tables after the C pass area: (rstd, -mean * rstd) per tile
-    // row, column sums of the tile's columns (written after the first pass barrier)
-    constexpr int TBL = PR * CST;
-    static_assert((TBL + 2 * MT + NT) * 4 <= NS * STAGE * 2, "LayerNorm tables fit the operand LDS");
-    float2* const ln_rt = (float2*)(Cs + TBL);
-    float* const ln_cs = Cs + TBL + 2 * MT;
     float badd[8], gadd[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) { badd[e] = 0.f; gadd[e] = 0.f; }
@@ -755,21 +711,9 @@ void gemm_kernel(GemmArgs a) {
     for (int sl = 0; sl < 2; ++sl)
 #pragma unroll
         for (int e = 0; e < 8; ++e) { st[sl][0][e] = 0.f; st[sl][1][e] = 0.f; }
-    // per-row output statistics (LayerNorm of the consumer): this thread's 8 columns
-    // of each of its rows
-    const bool do_rs = a.row_part != nullptr && !narrow;
-    float rsum[FM][MAXR], rsq[FM][MAXR];
-#pragma unroll
-    for (int ip = 0; ip < FM; ++ip)
-#pragma unroll
-        for (int k = 0; k < MAXR; ++k) { rsum[ip][k] = 0.f; rsq[ip][k] = 0.f; }
 #pragma unroll
     for (int ip = 0; ip < FM; ++ip) {
         __syncthreads();
-        if (lnc && ip == 0) {
-            if (tid % PPT == 0) ln_rt[tid / PPT] = ln_rs;
-            if (tid < NT) ln_cs[tid] = ln_cs_t;
-        }
         if constexpr (MF == 32) {
 #pragma unroll
         for (int j = 0; j < FN; ++j)
@@ -812,29 +756,14 @@ void gemm_kernel(GemmArgs a) {
             if (sr >= PR || m >= a.M) continue;
             // the row's 8 (GEGLU: 2 x 8) staged values as 16-byte LDS reads (rows are
             // CST = NT + 4 floats, tc a multiple of 8: 16-byte aligned)
-            // (LayerNorm consumer: rstd * (acc - mean * colsum) + bias)
             const float* crow = Cs + sr * CST + tc;
-            float2 lt = make_float2(1.f, 0.f);
-            if (lnc) lt = ln_rt[(sr >> 5) * TMW + ip * 32 + (sr & 31)];
             float v[8];
             ld8(crow, v);
-            if (lnc) {
-                float sn[8];
-                ld8(ln_cs + tc, sn);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = fmaf(lt.x, v[e], lt.y * sn[e]);
-            }
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] += badd[e];
             if (a.geglu) {
                 float g[8];
                 ld8(crow + 32, g);
-                if (lnc) {
-                    float sn[8];
-                    ld8(ln_cs + tc + 32, sn);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) g[e] = fmaf(lt.x, g[e], lt.y * sn[e]);
-                }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] *= gelu_erf(g[e] + gadd[e]);
             }
@@ -853,14 +782,6 @@ void gemm_kernel(GemmArgs a) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) oh[e] = (f16)v[e];
                 *(uint4*)((f16*)a.C + (int64_t)m * a.ldc + nout) = o;
-                if (do_rs) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float f = (float)oh[e];
-                        rsum[ip][k] += f;
-                        rsq[ip][k] += f * f;
-                    }
-                }
                 if (do_st) {
                     const bool s1 = m >= st_mb;
 #pragma unroll
@@ -880,25 +801,6 @@ void gemm_kernel(GemmArgs a) {
     if (do_st) {
         const int m_last = min(a.M, m0 + MT) - 1;
         stats_flush<NTH, NT / 8>(a, st, st_b0, m_last / a.stats_hw != st_b0 ? 2 : 1, n0, (float*)smem);
-    }
-    if (do_rs) {
-        // the cpr threads of a row are consecutive lanes, each 8 of them one 64-column
-        // group: add their partial sums; the first of the 8 stores the group's partial
-#pragma unroll
-        for (int ip = 0; ip < FM; ++ip)
-#pragma unroll
-            for (int k = 0; k < MAXR; ++k) {
-                float s1 = rsum[ip][k], s2 = rsq[ip][k];
-#pragma unroll
-                for (int off = 1; off < 8; off <<= 1) {
-                    s1 += __shfl_xor(s1, off);
-                    s2 += __shfl_xor(s2, off);
-                }
-                const int sr = r0 + k * rstep;
-                const int m = m0 + (sr >> 5) * TMW + ip * 32 + (sr & 31);
-                if ((oc & 63) == 0 && sr < PR && m < a.M && n < a.N)
-                    *(float2*)(a.row_part + ((int64_t)(n >> 6) * a.M + m) * 2) = make_float2(s1, s2);
-            }
     }
 }
 
@@ -996,7 +898,7 @@ struct Cfg {
     double t_fix;         // per-block prologue + epilogue time
     int spr;              // split slots per modelled round of the summing block's tail
     double conv_f;        // rate factor with the implicit-conv A (the tap gather)
-    int patch;            // conv3_patch_kernel's tile shape, or -1
+    int kind, shape;      // kernel, its tile shape
     double t_round;       // the summing block's time per modelled round
 };
 // 0: 256x128, 8 waves of 64x64, BK 64, 2-stage ring (96 KB: one block per CU)
@@ -1015,15 +917,23 @@ struct Cfg {
 // channels, batches 1 to 16, ragged sizes; every shape and split count timed): the planner's
 // choice is within 3% of the best of them on all but two (4%), and always a shape of
 // this kernel, so the convs it can take are planned among these alone.
-constexpr int kNumGemm = 4, kNumCfg = kNumGemm + kNumPatch;
-const Cfg kCfgs[kNumCfg] = {{256, 128, 1, 3.5e12, 3.5e12, 4.5e-6, 1, 1.0, -1, 0.9e-6},
-                            {128, 128, 2, 2.76e12, 3.9e12, 3.0e-6, 1, 1.0, -1, 0.9e-6},
-                            {128, 64, 2, 2.23e12, 3.03e12, 2.5e-6, 2, 0.8, -1, 0.9e-6},
-                            {64, 160, 2, 2.0e12, 3.4e12, 6.0e-6, 2, 0.9, -1, 0.9e-6},
-                            {256, 128, 1, 6.8e12, 6.8e12, 8.2e-6, 1, 1.0, 0, 1.0e-6},
-                            {256, 160, 1, 6.0e12, 6.0e12, 8.8e-6, 1, 1.0, 1, 1.2e-6},
-                            {128, 80, 2, 5.07e12, 5.2e12, 4.75e-6, 1, 1.0, 2, 0.39e-6},
-                            {128, 64, 2, 4.63e12, 5.08e12, 4.0e-6, 1, 1.0, 3, 0.33e-6}};
+// 8 ..: gemm_dense_kernel's shapes (k_dense.hip): 256x128 (8 waves, one block per CU),
+// 128x128, 128x64 (4 waves, two) and 64x64 (4 waves, three), fitted the same way to 2400
+// launches over 50 dense shapes (1 to 65536 rows, K 64 to 6400).
+enum Kind { K_GEMM = 0, K_PATCH = 1, K_DENSE = 2 };
+constexpr int kNumGemm = 4, kNumCfg = kNumGemm + kNumPatch + kNumDense;
+const Cfg kCfgs[kNumCfg] = {{256, 128, 1, 3.5e12, 3.5e12, 4.5e-6, 1, 1.0, K_GEMM, 0, 0.9e-6},
+                            {128, 128, 2, 2.76e12, 3.9e12, 3.0e-6, 1, 1.0, K_GEMM, 1, 0.9e-6},
+                            {128, 64, 2, 2.23e12, 3.03e12, 2.5e-6, 2, 0.8, K_GEMM, 2, 0.9e-6},
+                            {64, 160, 2, 2.0e12, 3.4e12, 6.0e-6, 2, 0.9, K_GEMM, 3, 0.9e-6},
+                            {256, 128, 1, 6.8e12, 6.8e12, 8.2e-6, 1, 1.0, K_PATCH, 0, 1.0e-6},
+                            {256, 160, 1, 6.0e12, 6.0e12, 8.8e-6, 1, 1.0, K_PATCH, 1, 1.2e-6},
+                            {128, 80, 2, 5.07e12, 5.2e12, 4.75e-6, 1, 1.0, K_PATCH, 2, 0.39e-6},
+                            {128, 64, 2, 4.63e12, 5.08e12, 4.0e-6, 1, 1.0, K_PATCH, 3, 0.33e-6},
+                            {256, 128, 1, 5.5e12, 5.5e12, 4.6e-6, 1, 1.0, K_DENSE, 0, 1.07e-6},
+                            {128, 128, 2, 3.76e12, 4.5e12, 3.1e-6, 1, 1.0, K_DENSE, 1, 0.97e-6},
+                            {128, 64, 2, 3.57e12, 3.8e12, 2.2e-6, 1, 1.0, K_DENSE, 2, 0.68e-6},
+                            {64, 64, 3, 2.04e12, 3.3e12, 1.4e-6, 1, 1.0, K_DENSE, 3, 0.44e-6}};
 // full kernel names, as the instantiations (tile configuration, A mode: 0 dense, 1 implicit conv,
 // then the MFMA)
 const char* const kNames[kNumGemm][2] = {{"gemm_kernel<256,128,4,2,64,2,0,32>", "gemm_kernel<256,128,4,2,64,2,1,32>"},
@@ -1036,21 +946,23 @@ int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // In-kernel split-K sum: tile counters at the head of the workspace (one per tile).
 constexpr int kMaxSplitTiles = 16384;
 constexpr size_t kCounterBytes = kMaxSplitTiles * sizeof(unsigned);
-// Split costs outside the kernels' own time, for gemm_kernel and conv3_patch_kernel: the fp32
+// Split costs outside the kernels' own time, by kernel, from the same fits: the fp32
 // partial round trip's rate (mostly L2 / Infinity Cache resident), the in-kernel sum's fixed
 // part, the reduce launch.
 struct SplitCost {
     double rate, fix, red;
-};
-constexpr SplitCost kSplit[2] = {{20.0e12, 1.0e-6, 5.5e-6}, {38.0e12, 2.9e-6, 4.2e-6}};
+};  // by Kind
+constexpr SplitCost kSplit[3] = {{20.0e12, 1.0e-6, 5.5e-6}, {38.0e12, 2.9e-6, 4.2e-6}, {12.0e12, 0.3e-6, 4.5e-6}};
 
-const char* cfg_name(int ci, const GemmArgs& a) {
-    return ci < kNumGemm ? kNames[ci][a.amode == A_CONV3] : conv_patch_name(kCfgs[ci].patch, a.subpix);
+std::string cfg_name(int ci, const GemmArgs& a) {
+    const Cfg& g = kCfgs[ci];
+    if (g.kind == K_DENSE) return dense_name(g.shape, a);
+    return g.kind == K_GEMM ? kNames[ci][a.amode == A_CONV3] : conv_patch_name(g.shape, a.subpix);
 }
 
 int cfg_tiles(int ci, const GemmArgs& a) {
-    const int tm = ci < kNumGemm ? ceil_div(a.M, kCfgs[ci].mt) : conv_patch_tiles_m(kCfgs[ci].patch, a);
-    return tm * ceil_div(a.N, kCfgs[ci].nt);
+    const Cfg& g = kCfgs[ci];
+    return (g.kind == K_PATCH ? conv_patch_tiles_m(g.shape, a) : ceil_div(a.M, g.mt)) * ceil_div(a.N, g.nt);
 }
 
 // The convs the patch-resident kernel takes.  (Pixel indices stay below 2^24: 64 channels of
@@ -1071,26 +983,20 @@ bool stats_tile_ok(int mt, int hw) { return hw >= mt || mt == 2 * hw; }
 // partial round trip and the serial tail of the block that sums a tile's partials, or
 // the reduce launch.
 void plan(const GemmArgs& a, int& ci, int& splits, int& kps, bool& fix) {
-    const bool patch = patch_ok(a);
+    const int kind = patch_ok(a) ? K_PATCH : dense_ok(a) ? K_DENSE : K_GEMM;
+    const bool patch = kind == K_PATCH;
     const int nkt = ceil_div(a.K, 64), nc = patch ? a.Cin / 64 : 0, ntap = a.subpix ? 4 : 9;
     double best = 1e30;
-    ci = patch ? kNumGemm : 1; splits = 1; kps = nkt * 64; fix = false;
-    for (int c = patch ? kNumGemm : 0; c < (patch ? kNumCfg : kNumGemm); ++c) {
+    ci = 1; splits = 1; kps = nkt * 64; fix = false;
+    for (int c = 0; c < kNumCfg; ++c) {
         const Cfg& g = kCfgs[c];
-        if (patch) {
-            if (a.subpix && !conv_patch_subpix(g.patch)) continue;
-        } else {
+        if (g.kind != kind || (a.subpix && !conv_patch_subpix(g.shape))) continue;
+        if (kind == K_GEMM) {
             if (a.geglu && g.nt % 128) continue;  // GEGLU pairs 32-column blocks within a 64-wide wave tile
-            // LayerNorm row partials: one per 64 columns, summed by 8 consecutive lanes
-            if (a.row_part && g.nt % 64) continue;
-            // the LayerNorm consumer's epilogue runs 5-8% slower in the 4-wave 64x160 tile than
-            // the 128x128 tile at K = 1280 (M = 1152, N = 3840: 27.8 against 25.7 us), which
-            // the model does not see
-            if (a.ln_part && g.mt == 64) continue;
             if (a.stats && !stats_tile_ok(g.mt, a.stats_hw)) continue;
         }
         const int tiles = cfg_tiles(c, a);
-        const SplitCost& sc = kSplit[patch];
+        const SplitCost& sc = kSplit[kind];
         static const int cand[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
         for (int s : cand) {
             if (s > 1 && nkt / s < 4) break;
@@ -1116,7 +1022,7 @@ void plan(const GemmArgs& a, int& ci, int& splits, int& kps, bool& fix) {
                 fx = t_fix < t_red;
                 t += fx ? t_fix : t_red;
             }
-            if (t < best * (patch ? 0.999 : 0.98)) { best = t; ci = c; splits = se; kps = kt_per * 64; fix = fx; }
+            if (t < best * (kind == K_GEMM ? 0.98 : 0.999)) { best = t; ci = c; splits = se; kps = kt_per * 64; fix = fx; }
         }
     }
 }
@@ -1124,7 +1030,7 @@ void plan(const GemmArgs& a, int& ci, int& splits, int& kps, bool& fix) {
 
 bool gemm_stats_supported(int hw) { return stats_tile_ok(128, hw); }
 
-const char* gemm_kernel_name(const GemmArgs& a) {
+std::string gemm_kernel_name(const GemmArgs& a) {
     if (narrow_conv(a)) return a.N <= 4 ? "conv3_narrow_kernel<4>" : "conv3_narrow_kernel<8>";
     int ci, splits, kps;
     bool fix;
@@ -1180,9 +1086,10 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
     if (a.A3 == nullptr) a.K2 = a.K;
     const Cfg& g = kCfgs[ci];
     // a conv's dense tail and the sub-pixel form are the patch kernel's
-    if ((a.A3 && (a.amode != A_CONV3 || !a.A2)) || ((a.subpix || (a.amode == A_CONV3 && a.A2)) && g.patch < 0))
+    if ((a.A3 && (a.amode != A_CONV3 || !a.A2)) || ((a.subpix || (a.amode == A_CONV3 && a.A2)) && g.kind != K_PATCH))
         return hipErrorInvalidValue;
-    // (a consumer thread sums up to 10 row partials; 2 or 4 threads per tile row)
+    // the LayerNorm forms are the dense kernel's
+    if ((a.ln_part || a.row_part) && g.kind != K_DENSE) return hipErrorInvalidValue;
     if (a.ln_part && (a.amode != A_DENSE || a.A2 || !a.ln_colsum || a.out_mode != OUT_F16 || (a.N & 7) ||
                       (a.K & 63) || a.K > 1280 || !(a.ln_eps > 0.f) || (splits > 1 && !fix)))
         return hipErrorInvalidValue;
@@ -1192,7 +1099,7 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
         if (a.A2 || a.K != 4 * a.Cin || a.Ho != 2 * a.Hin || a.Wo != 2 * a.Win || a.M != a.Bn * a.Ho * a.Wo || a.res ||
             a.out_mode != OUT_F16 || (splits > 1 && !fix))
             return hipErrorInvalidValue;
-    } else if (g.patch >= 0) {
+    } else if (g.kind == K_PATCH) {
         if (a.K1 != 9 * a.Cin || a.Ho != a.Hin || a.Wo != a.Win || a.M != a.Bn * a.Ho * a.Wo) return hipErrorInvalidValue;
     }
     if (a.amode == A_CONV3 && a.A2 &&
@@ -1222,7 +1129,7 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
                                (a.A2 && 2 * (int64_t)a.M * a.lda2 > lim) || (a.A3 && 2 * (int64_t)a.M * a.lda3 > lim)))
         return hipErrorInvalidValue;
     if (a.stats && (a.out_mode != OUT_F16 || a.geglu || (a.N & 7) || a.stats_hw < 64 ||
-                    (g.patch < 0 ? !stats_tile_ok(g.mt, a.stats_hw) : a.stats_hw != a.Ho * a.Wo)))
+                    (g.kind == K_GEMM ? !stats_tile_ok(g.mt, a.stats_hw) : g.kind == K_PATCH && a.stats_hw != a.Ho * a.Wo)))
         return hipErrorInvalidValue;
     const dim3 grid(cfg_tiles(ci, a), 1, splits);
     // algorithmic traffic: A once (the conv source image, not its im2col), W once, output
@@ -1238,8 +1145,9 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
     const double kop = a.subpix ? 9.0 * a.Cin : (double)a.K;
     const double flops = 2.0 * a.M * a.N * kop;
     const double k_bytes = a_bytes + 2.0 * a.N * kop + out_bytes;
-    launch_timed(cfg_name(ci, a), flops, k_bytes, [&] {
-        if (g.patch >= 0) conv_patch_launch(g.patch, a, s);
+    launch_timed(cfg_name(ci, a).c_str(), flops, k_bytes, [&] {
+        if (g.kind == K_PATCH) conv_patch_launch(g.shape, a, s);
+        else if (g.kind == K_DENSE) dense_launch(g.shape, a, s);
         else if (a.amode == A_DENSE) launch_cfg<A_DENSE>(ci, grid, a, s);
         else launch_cfg<A_CONV3>(ci, grid, a, s);
     });

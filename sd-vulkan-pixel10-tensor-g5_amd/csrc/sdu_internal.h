@@ -8,21 +8,24 @@
 
 #include <cstdint>
 #include <cstddef>
+#include <string>
 
 namespace sdu {
 
 typedef _Float16 f16;
 
-// GELU with the erf of Abramowitz & Stegun 7.1.26 (|error| <= 1.5e-7): the branch-free
-// form the reference's geglu_f32.comp evaluates, gelu(x) = 0.5 x (1 + erf(x / sqrt 2)).
-__device__ __forceinline__ float erf_as(float x) {
+// GELU with the erf of Abramowitz & Stegun 7.1.26 (|error| <= 1.5e-7), the branch-free form the
+// reference's geglu_f32.comp evaluates.  With erf(z) = 1 - p(t) exp(-z^2), t = 1 / (1 + c z),
+// z = |x| / sqrt 2: 0.5 x (1 + erf(x / sqrt 2)) = max(x, 0) - |x| (p(t) / 2) exp(-x^2 / 2),
+// the same for both signs, with the constant factors folded into the polynomial.
+__device__ __forceinline__ float gelu_erf(float x) {
     const float ax = fabsf(x);
-    const float t = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * ax);
-    const float p = ((((1.061405429f * t - 1.453152027f) * t + 1.421413741f) * t - 0.284496736f) * t +
-                     0.254829592f) * t;
-    return copysignf(1.0f - p * __expf(-ax * ax), x);
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f * 0.70710678118654752f, ax, 1.0f));
+    const float e = __builtin_amdgcn_exp2f(x * (x * -0.72134752044448170f));
+    const float p = fmaf(fmaf(fmaf(fmaf(0.5f * 1.061405429f, t, 0.5f * -1.453152027f), t, 0.5f * 1.421413741f), t,
+                              0.5f * -0.284496736f), t, 0.5f * 0.254829592f) * t;
+    return fmaf(-fminf(ax, 3.4e38f), p * e, fmaxf(x, 0.f));  // (a finite factor: x = inf gives inf)
 }
-__device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.0f + erf_as(x * 0.70710678118654752f)); }
 
 // ----------------------------------------------------------------- kernel timing
 // Eager profiling hook.  While a KernelTimer is installed on the calling thread
@@ -157,7 +160,7 @@ bool gemm_stats_supported(int hw);
 // be zero before the first launch on a workspace and every launch leaves them zero.
 size_t gemm_counter_bytes();
 size_t gemm_workspace_bytes(const GemmArgs& a);
-const char* gemm_kernel_name(const GemmArgs& a);  // tile variant the launch will use
+std::string gemm_kernel_name(const GemmArgs& a);  // tile variant the launch will use
 hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s);
 // Sum a.splits fp32 partials [splits][M][N] at a.partial and run the epilogue.
 hipError_t splitk_reduce_launch(const GemmArgs& a, double bytes, hipStream_t s);
@@ -169,6 +172,12 @@ int conv_patch_tiles_m(int cfg, const GemmArgs& a);
 bool conv_patch_subpix(int cfg);  // the shape has a sub-pixel form
 const char* conv_patch_name(int cfg, bool subpix);
 void conv_patch_launch(int cfg, const GemmArgs& a, hipStream_t s);
+// The dense GEMM kernel with the register epilogue (k_dense.hip): tile shape `cfg` of
+// kNumDense, for the GEMMs dense_ok takes.
+constexpr int kNumDense = 4;
+bool dense_ok(const GemmArgs& a);
+std::string dense_name(int cfg, const GemmArgs& a);
+void dense_launch(int cfg, const GemmArgs& a, hipStream_t s);
 // Sub-pixel weights of a 3x3 conv that follows a 2x nearest upsampling (GemmArgs::subpix):
 // w3 [Cout][3][3][Cin] -> w4 [4 phases][Cout][2][2][Cin], phase = 2 py + px.  Tap (ty, tx)
 // of phase (py, px) is the fp32 sum of the 3x3 taps (ky, kx) with ty = (py + ky + 1) / 2 - py

@@ -227,6 +227,42 @@ def test_matmul(op_engine, M, N, K, K2, bias, res, geglu, f32):
     assert np.abs(got - ref).max() < 3e-2 * max(1.0, np.abs(ref).max() / 8)
 
 
+@pytest.mark.parametrize("M,N,K,K2,bias,res,geglu,f32", [
+    (1, 8, 64, 0, True, True, False, False),          # one row, one 8-column chunk, one K step
+    (63, 72, 128, 0, True, False, False, True),       # a row short of a tile, 8 columns past one
+    (65, 64, 192, 64, False, True, False, False),     # a row past a tile, second source after 2 steps
+    (129, 136, 64, 0, True, True, False, False),
+    (257, 192, 320, 0, True, False, True, False),     # GEGLU, N not a multiple of the wide tiles
+    (40000, 136, 64, 0, True, True, False, False),    # several tiles per persistent block, one K step each
+    (33000, 320, 128, 64, True, False, False, False),  # the same, two sources of one step each
+    (20000, 640, 192, 0, True, False, True, False),   # the same, GEGLU
+    (70, 72, 2048, 0, True, True, False, False),      # split K over ragged tiles
+    (300, 200, 4096, 1024, True, True, False, False),  # split K whose later blocks start in the second source
+])
+def test_matmul_dense_tiles(op_engine, M, N, K, K2, bias, res, geglu, f32):
+    """Edges of the dense kernel's tiles and of its persistent blocks' tile hand-over."""
+    test_matmul(op_engine, M, N, K, K2, bias, res, geglu, f32)
+
+
+def test_geglu_gate_range(op_engine):
+    """The gate's GELU over fp16's range: exact zero below about -6, the identity above, infinity
+    kept.  A&S 7.1.26's 1.5e-7 on erf bounds the absolute error by 7.5e-8 |b|; the rest is the
+    output's fp16 rounding (2^-11 relative, 2^-25 below the normal range)."""
+    e = op_engine
+    b = np.concatenate([np.linspace(-8, 8, 4001), [-65504, -300, 300, 65504, 0.0, -0.0, 6e-8, -6e-8, np.inf]]).astype(np.float16)
+    a = np.where(np.arange(b.size) % 2, 0.75, -1.0).astype(np.float16)
+    a[np.abs(b) > 100] = 1.0
+    ty = e.tensor((1, b.size))
+    e.geglu(e.upload(np.concatenate([a, b])[None]), ty, 1, b.size)
+    got = ty.numpy()[0].astype(np.float64)
+    bd = t(b.astype(np.float64))
+    ref = (t(a.astype(np.float64)) * (bd * 0.5 * torch.erfc(-bd / math.sqrt(2.0)))).numpy()
+    assert np.isposinf(got[-1]) and np.isposinf(ref[-1])
+    got, ref, g = got[:-1], ref[:-1], np.abs(b[:-1].astype(np.float64))
+    err, r = np.abs(got - ref), np.abs(ref)
+    assert (err <= r * 2.0**-11 + 2.0**-25 + 1e-7 * g).all()
+
+
 def test_matmul_split_repeat(op_engine):
     """Split-K launches back to back: the per-tile arrival counters are left zero by
     each launch, and the tile sums run in a fixed order, so repeats are bit-identical."""
