@@ -121,14 +121,14 @@ int op_gemm(sdu_ctx* ctx, const GemmArgs& g, const char* what) {
 }
 
 // ---- scratch of the no-allocation GroupNorm (sdu_groupnorm_noalloc)
-// The fp64 per-(image, group) sums and sums of squares of the GroupNorm statistics pass
-// live in this file-scope device array instead of the context's allocated workspace:
-// 64 images x 32 groups x 2 = 32 KiB, held by every device the library runs on until
-// the process ends.  In host code `scratch` is only a symbol: its device address is
+// The partial sums of the GroupNorm statistics pass live in this file-scope device array
+// instead of the context's allocated workspace: 64 KiB (groupnorm_acc_bytes is at most that
+// for images x groups <= 64 x 32), held by every device the library runs on until the
+// process ends.  In host code `scratch` is only a symbol: its device address is
 // resolved once per device (hipGetSymbolAddress, with that device current) at sdu_init
 // and every host use goes through that address.
 constexpr int kNoAllocMaxB = 64, kNoAllocMaxG = 32;
-constexpr size_t kNoAllocScratchBytes = (size_t)kNoAllocMaxB * kNoAllocMaxG * 2 * sizeof(double);
+constexpr size_t kNoAllocScratchBytes = 64 * 1024;
 static __device__ __align__(256) double scratch[kNoAllocScratchBytes / sizeof(double)];
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -773,11 +773,9 @@ int sdu_groupnorm(sdu_ctx* ctx, const sdu_tensor* x, const sdu_tensor* x2, const
     const size_t acc = groupnorm_acc_bytes(B, groups);
     st = ensure_op_ws(ctx->c, acc);
     if (st) return st;
-    hipError_t e = zero_launch(ctx->c.op_ws, acc, ctx->c.stream);
-    if (e == hipSuccess)
-        e = groupnorm_launch((const f16*)dptr(x), (const f16*)dptr(x2), C1, C2, (const f16*)dptr(gamma),
-                             (const f16*)dptr(beta), (f16*)dptr(y), B, HW, groups, eps, silu,
-                             (double*)ctx->c.op_ws, ctx->c.stream);
+    const hipError_t e =
+        groupnorm_launch((const f16*)dptr(x), (const f16*)dptr(x2), C1, C2, (const f16*)dptr(gamma),
+                         (const f16*)dptr(beta), (f16*)dptr(y), B, HW, groups, eps, silu, ctx->c.op_ws, ctx->c.stream);
     return finish(ctx, e, "groupnorm");
 }
 
@@ -788,17 +786,13 @@ int sdu_groupnorm_noalloc(sdu_ctx* ctx, const sdu_tensor* x, const sdu_tensor* x
     OpTimerScope ots(ctx, "groupnorm_noalloc");
     int st = gn_check(ctx, x, x2, gamma, beta, y, B, HW, C1, C2, groups);
     if (st) return st;
-    const size_t acc = groupnorm_acc_bytes(B, groups);
-    if (acc > kNoAllocScratchBytes)
-        return fail(ctx, SDU_ERR_ARG, "groupnorm_noalloc: images x groups exceed the 32 KiB scratch (64 x 32)");
+    if ((size_t)B * groups > kNoAllocMaxB * kNoAllocMaxG || groupnorm_acc_bytes(B, groups) > kNoAllocScratchBytes)
+        return fail(ctx, SDU_ERR_ARG, "groupnorm_noalloc: images x groups exceed the scratch (64 x 32)");
     void* p = scratch_addr(ctx->c.device);
     if (!p) return fail(ctx, SDU_ERR_HIP, "groupnorm_noalloc: scratch address not resolved for this device");
-    // the statistics pass accumulates into the scratch: clear it with a fill kernel first
-    hipError_t e = zero_launch(p, acc, ctx->c.stream);
-    if (e == hipSuccess)
-        e = groupnorm_launch((const f16*)dptr(x), (const f16*)dptr(x2), C1, C2, (const f16*)dptr(gamma),
-                             (const f16*)dptr(beta), (f16*)dptr(y), B, HW, groups, eps, silu, (double*)p,
-                             ctx->c.stream);
+    const hipError_t e = groupnorm_launch((const f16*)dptr(x), (const f16*)dptr(x2), C1, C2, (const f16*)dptr(gamma),
+                                          (const f16*)dptr(beta), (f16*)dptr(y), B, HW, groups, eps, silu, p,
+                                          ctx->c.stream);
     return finish(ctx, e, "groupnorm_noalloc");
 }
 

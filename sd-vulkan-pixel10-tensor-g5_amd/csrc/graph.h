@@ -47,7 +47,7 @@ struct Exec {
     bool dry = false;
     float* gemm_ws = nullptr;
     size_t gemm_ws_need = 0;
-    double* gn_acc = nullptr;  // next free GroupNorm accumulator slot (zeroed per forward)
+    void* gn_acc = nullptr;     // GroupNorm scratch (groupnorm_acc_bytes), one launch at a time
     double* st_next = nullptr;  // per-channel output statistics pool (zeroed per forward)
     double* st_end = nullptr;
     // A forward clears its statistics pool in the launch that stages its inputs, outside
@@ -131,7 +131,7 @@ inline void want_stats(Exec& E, GemmArgs& a, int HW) {
 
 // GroupNorm (32 groups, epsilon eps) of concat(x, x2) over C1 + C2 channels, optionally
 // followed by SiLU: from the producers' epilogue statistics when both kept them, else
-// with its own statistics pass (accumulator slot from E.gn_acc).
+// with its own statistics pass.
 inline void group_norm_op(Exec& E, Act x, Act x2, int C1, int C2, const f16* g, const f16* b, f16* y, int HW,
                           int silu, float eps) {
     const int G = 32;
@@ -144,10 +144,8 @@ inline void group_norm_op(Exec& E, Act x, Act x2, int C1, int C2, const f16* g, 
         }, shape);
         return;
     }
-    double* acc = E.gn_acc;
-    E.gn_acc += (size_t)E.B * G * 2;
     E.run(silu ? "groupnorm_silu" : "groupnorm", [&] {
-        return groupnorm_launch(x.p, x2.p, C1, C2, g, b, y, E.B, HW, G, eps, silu, acc, E.s);
+        return groupnorm_launch(x.p, x2.p, C1, C2, g, b, y, E.B, HW, G, eps, silu, E.gn_acc, E.s);
     }, shape);
 }
 

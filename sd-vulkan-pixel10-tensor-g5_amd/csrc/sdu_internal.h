@@ -210,12 +210,12 @@ hipError_t attention_launch(const AttnArgs& a, hipStream_t s);
 size_t attention_workspace_bytes(const AttnArgs& a);
 
 // ----------------------------------------------------------------- norms
-// GroupNorm accumulator: fp64 [B][G][2] (sum, sum of squares); must be zero on
-// entry (zero_launch).  C = C1 + C2 <= 2560, G <= 32.
+// acc: scratch of groupnorm_acc_bytes, nothing kept in it between launches (the statistics
+// pass's partial sums).  C = C1 + C2 <= 2560, G <= 32.
 size_t groupnorm_acc_bytes(int B, int G);
 hipError_t groupnorm_launch(const f16* x, const f16* x2, int C1, int C2, const f16* gamma,
                             const f16* beta, f16* y, int B, int HW, int G, float eps, int silu,
-                            double* acc, hipStream_t s);
+                            void* acc, hipStream_t s);
 // GroupNorm apply from per-channel statistics produced by the GEMMs that wrote x and
 // x2 (GemmArgs::stats: [B][C1][2] and [B][C2][2] fp64 sums and sums of squares).
 hipError_t groupnorm_apply_stats_launch(const f16* x, const f16* x2, int C1, int C2, const double* st1,

@@ -239,26 +239,22 @@ static void unet_core(Exec& E, const Fwd& F, const f16* lat, const float* temb32
                       float* out, const float* tproj_pre = nullptr, void* const* out_ind = nullptr) {
     Ctx& c = E.c;
     const size_t mk0 = E.ar->mark();
-    // GroupNorm accumulators of this forward (2 per resnet, 1 per transformer, conv_norm_out)
-    // for GroupNorms that compute their own statistics, then the pool of per-channel
+    // scratch of the GroupNorms that compute their own statistics, and the pool of per-channel
     // statistics of the GEMM outputs that GroupNorms read (conv1 and conv2 of every
-    // resnet, every transformer's proj_out, conv_in and the 6 resampling convs);
-    // one clear for both.
-    const size_t n_gn = 2 * c.resnets.size() + c.xfs.size() + 1;
-    const size_t acc_n = n_gn * groupnorm_acc_bytes(E.B, kGroups) / sizeof(double);
+    // resnet, every transformer's proj_out, conv_in and the 6 resampling convs), cleared once
     size_t st_ch = 7 * 1280;
     for (const ResDesc& r : c.resnets) st_ch += 2 * r.cout;
     for (const XfDesc& t : c.xfs) st_ch += t.c;
     const size_t st_n = (size_t)E.B * st_ch * 2;
-    E.gn_acc = E.alloc<double>(acc_n + st_n);
-    E.st_next = E.gn_acc + acc_n;
+    E.gn_acc = E.alloc<char>(groupnorm_acc_bytes(E.B, kGroups));
+    E.st_next = E.alloc<double>(st_n);
     E.st_end = E.st_next + st_n;
     if (E.stats_outside) {
-        E.stats_pool = E.gn_acc;
-        E.stats_bytes = (acc_n + st_n) * sizeof(double);
+        E.stats_pool = E.st_next;
+        E.stats_bytes = st_n * sizeof(double);
     } else {
-        void* p = E.gn_acc;
-        E.run("groupnorm", [&] { return zero_launch(p, (acc_n + st_n) * sizeof(double), E.s); });
+        void* p = E.st_next;
+        E.run("groupnorm", [&] { return zero_launch(p, st_n * sizeof(double), E.s); });
     }
     const float* tproj = tproj_pre ? tproj_pre : time_embed(E, temb320);
     int H = F.H, Wd = F.W;

@@ -271,17 +271,15 @@ static Act attention(Exec& E, AuxNet& n, Act x, int H, int W) {
 static void vae_body(Exec& E, AuxNet& n, AuxState& S) {
     const int B = S.key[0];
     int h = S.key[1], w = S.key[2];
-    // GroupNorm accumulators (2 per resnet, the attention's, conv_norm_out) and the
-    // statistics pool of the GEMM outputs GroupNorms read, cleared by one fill kernel
-    const size_t n_gn = 2 * 14 + 2;
-    const size_t acc_n = n_gn * groupnorm_acc_bytes(B, 32) / sizeof(double);
+    // GroupNorm scratch and the statistics pool of the GEMM outputs GroupNorms read, cleared
+    // by a fill kernel
     const size_t st_n = (size_t)B * 40 * kTop * 2;
-    E.gn_acc = E.alloc<double>(acc_n + st_n);
-    E.st_next = E.gn_acc + acc_n;
+    E.gn_acc = E.alloc<char>(groupnorm_acc_bytes(B, 32));
+    E.st_next = E.alloc<double>(st_n);
     E.st_end = E.st_next + st_n;
     {
-        void* pool = E.gn_acc;
-        E.run("vae_io", [&] { return zero_launch(pool, (acc_n + st_n) * sizeof(double), E.s); });
+        void* pool = E.st_next;
+        E.run("vae_io", [&] { return zero_launch(pool, st_n * sizeof(double), E.s); });
     }
     f16* x0 = E.alloc<f16>((size_t)B * h * w * 8);
     E.run("vae_io", [&] {

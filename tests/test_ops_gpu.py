@@ -62,6 +62,20 @@ def test_groupnorm(op_engine, B, H, W, C1, C2, silu):
     assert np.array_equal(ty.numpy().astype(np.float32), got)
 
 
+@pytest.mark.parametrize("B,H,W,C1,C2,silu", [
+    (1, 1, 1, 96, 0, False),          # one pixel: one block, one phase of 42
+    (3, 1, 41, 32, 64, True),         # a pixel short of a block's phases, concat inside a group
+    (64, 3, 3, 96, 0, True),          # the largest batch: 4 statistics blocks per image
+    (1, 97, 31, 2560, 0, True),       # one pixel phase, ragged last block
+    (2, 131, 67, 256, 288, True),     # 68 octets: idle threads in every block
+    (1, 257, 263, 32, 0, False),      # one channel per group, several rounds per thread
+])
+def test_groupnorm_two_pass(op_engine, B, H, W, C1, C2, silu):
+    """Edges of the statistics and apply passes' blocks (3 channels per group, or slabs above 64K
+    elements: beyond the single-kernel form)."""
+    test_groupnorm(op_engine, B, H, W, C1, C2, silu)
+
+
 @pytest.mark.parametrize("B,H,W,C,silu", [(2, 32, 32, 640, True), (2, 16, 16, 1280, False)])
 def test_groupnorm_large_mean(op_engine, B, H, W, C, silu):
     """Groups whose mean is 100x their spread (the single-kernel path sums x minus the
