@@ -24,15 +24,18 @@
 // the shared-tile kernel also moves the FMA into the MFMA: that dimension of Q holds
 // -m against a K column of ones, so the scores come out as s*c - m (ofs_update).
 //
-// Two kernels:
+// Three kernels:
 //   attn_kernel       -- NWAVE query waves share each 64-key K/V tile in LDS
 //                        (long sequences: 64x64 self-attention, 4096 tokens);
+//   attn_wide_kernel  -- the same with 64 queries per wave, scores of the next keys formed
+//                        during the softmax of these (many query blocks, heads of 33..64);
 //   attn_split_kernel -- NSPLIT waves split the keys of one 32-query group and
 //                        merge their partial (max, sum, O) through LDS (short query
 //                        counts, where one wave per 32 queries cannot fill the chip).
 #include "sdu_internal.h"
 
 #include <cstdio>
+#include <type_traits>
 
 namespace sdu {
 
@@ -507,6 +510,286 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_kernel(AttnArgs a) {
     }
 }
 
+// ----------------------------------------------------------------- wide shared-tile kernel
+
+// 64 queries per wave (two groups of 32 that share every K and V fragment read), 4 waves per block,
+// 64-key tiles through a ring of three.  KS, MTD, LSUM and OFS as in attn_kernel.
+//
+// Bound by VALU issue: a wave's 32-key step is 14 MFMAs (448 cycles at d 40) beside 32 v_exp_f32 (8
+// cycles each, 10 from a lone wave), 16 converts and 16-20 max, and an MFMA takes some 10
+// cycles of VALU issue.  In attn_kernel the two mostly took turns, every fragment was read from
+// LDS for 32 queries only (as many LDS cycles as MFMA cycles), and each tile's scores, max and
+// exps waited for one another.  Here the scores of the next 32 keys are formed among the
+// exps of this one's, and their max among its PV products: one straight line of code, the
+// order set by sched_group_barrier, one branch (the reference moves) at its end.
+// d 40, 16 heads x images: 4096 tokens 81 -> 67 us (scale applied in the softmax), 77 -> 62
+// (q pre-scaled); 128 heads x images 513 -> 433 us.
+template <int KS, int MTD, bool LSUM, bool OFS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn_wide_kernel(AttnArgs a) {
+    constexpr int KT = 64, G = 2;
+    constexpr int VSTR = ((MTD * 32 - 16 + 63) / 64) * 64 + 16;  // as attn_kernel's TRV
+    constexpr int KSTR = KS * 16 + 8, KTILE = KT * KSTR, VTILE = KT * VSTR, NTH = 256;
+    __shared__ __attribute__((aligned(16))) f16 Ks[3 * KTILE];
+    __shared__ __attribute__((aligned(16))) f16 Vs[3 * VTILE];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = blockIdx.y, b = blockIdx.z;
+    const int d = a.d, dch = d >> 3;
+    const int q0 = blockIdx.x * 256 + wave * 64;
+    const int lrow = lane & 31, hl = lane >> 5, lk = hl * 8;
+    const float c = a.q_log2 ? 1.f : a.scale * 1.4426950408889634f;
+
+    // K columns [d, KS*16) (OFS: column d is 1) and V dims [d, MTD*32) (LSUM: the last is 1),
+    // never overwritten by the tile stores
+    for (int i = tid; i < 3 * KT; i += NTH)
+        for (int x = d; x < KS * 16; ++x) Ks[i * KSTR + x] = (f16)((OFS && x == d) ? 1.f : 0.f);
+    for (int i = tid; i < 3 * KT; i += NTH)
+        for (int x = d; x < MTD * 32; ++x) Vs[i * VSTR + x] = (f16)((LSUM && x == MTD * 32 - 1) ? 1.f : 0.f);
+
+    half8 qf[G][KS];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const int q = q0 + g * 32 + lrow;
+        const f16* qp = a.q + ((int64_t)b * a.Sq + q) * a.ldq + (int64_t)h * d;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int dd = ks * 16 + lk;
+            half8 v = {};
+            if (q < a.Sq && dd < d) v = *(const half8*)(qp + dd);
+            qf[g][ks] = v;
+        }
+    }
+
+    // tile loads as in attn_kernel: rows past Sk and threads without a chunk read zeros
+    const f16* kbase = a.k + (int64_t)b * a.Sk * a.ldk + (int64_t)h * d;
+    const f16* vbase = a.v + (int64_t)b * a.Sk * a.ldv + (int64_t)h * d;
+    const __amdgpu_buffer_rsrc_t rsk =
+        __builtin_amdgcn_make_buffer_rsrc((void*)kbase, (short)0, ((a.Sk - 1) * a.ldk + d) * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsv =
+        __builtin_amdgcn_make_buffer_rsrc((void*)vbase, (short)0, ((a.Sk - 1) * a.ldv + d) * 2, 0x00020000);
+    constexpr int MAXCH = (KT * KS * 2 + NTH - 1) / NTH;
+    uint4 rk[MAXCH], rv[MAXCH];
+    uint32_t kvo[MAXCH], vvo[MAXCH];
+    int sto[MAXCH], vto[MAXCH];  // LDS offsets (halves) in the tile; -1: no chunk
+#pragma unroll
+    for (int i = 0; i < MAXCH; ++i) {
+        const int ci = tid + i * NTH, key = ci / dch, dc = ci - key * dch;
+        const bool ok = ci < KT * dch;
+        kvo[i] = ok ? (uint32_t)((key * a.ldk + dc * 8) * 2) : 0x80000000u;
+        vvo[i] = ok ? (uint32_t)((key * a.ldv + dc * 8) * 2) : 0x80000000u;
+        sto[i] = ok ? key * KSTR + dc * 8 : -1;
+        vto[i] = ok ? key * VSTR + dc * 8 : -1;
+    }
+    const uint32_t kstep = (uint32_t)(KT * a.ldk * 2), vstep = (uint32_t)(KT * a.ldv * 2);
+    auto load_kv = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MAXCH; ++i) {
+            rk[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsk, kvo[i], 0, 0));
+            rv[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsv, vvo[i], 0, 0));
+            kvo[i] += kstep;
+            vvo[i] += vstep;
+        }
+    };
+    auto store_kv = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MAXCH; ++i)
+            if (sto[i] >= 0) {
+                *(uint4*)&Ks[buf * KTILE + sto[i]] = rk[i];
+                *(uint4*)&Vs[buf * VTILE + vto[i]] = rv[i];
+            }
+    };
+
+    load_kv();
+    __syncthreads();  // padding set before the first tile stores land next to it
+    store_kv(0);
+    load_kv();
+    store_kv(1);
+    load_kv();
+    __syncthreads();
+
+    floatx16 o[G][MTD];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int t = 0; t < MTD; ++t) o[g][t] = floatx16{};
+    // the reference; !OFS: less it (0 for none yet, as softmax_pv) and the raw score that moves it
+    float m_run[G], l_run[G], nm[G], thr[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) { m_run[g] = OFS ? 0.f : -INFINITY; l_run[g] = nm[g] = thr[g] = 0.f; }
+    const float inv_c = 1.f / c;
+
+    const int vlo = tr_lane_offset(lane, VSTR), klo = key_perm(lrow) * KSTR + lk;
+    half8 kf[KS];
+    auto load_kf = [&](const f16* kt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) kf[ks] = *(const half8*)(kt + ks * 16);
+    };
+    auto qk = [&](floatx16 (&s)[G]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) s[g] = floatx16{};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int g = 0; g < G; ++g) s[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[g][ks], s[g], 0, 0, 0);
+    };
+    // (element e of lane half hl is key 16 (e / 8) + 8 hl + e % 8, see key_perm)
+    auto mask = [&](floatx16 (&s)[G], int kv) __attribute__((always_inline)) {
+        const int kl = kv - 8 * hl;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+#pragma unroll
+            for (int g = 0; g < G; ++g) s[g][e] = 16 * (e >> 3) + (e & 7) < kl ? s[g][e] : -INFINITY;
+    };
+    // The lane's own max of each group's scores (the other half of its query's keys is in lane ^ 32).
+    auto lane_max = [&](const floatx16 (&s)[G], float (&mx)[G]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            mx[g] = s[g][0];
+#pragma unroll
+            for (int e = 1; e < 16; ++e) mx[g] = fmaxf(mx[g], s[g][e]);
+        }
+    };
+    // Moves the softmax references up to the scores s (wave-uniformly rare, see softmax_pv and
+    // ofs_update): O and the row sums are rescaled; OFS: s, which carries the old reference, too,
+    // and Q's spare dimension takes the new one for the sub-tiles to come.
+    auto rebase = [&](floatx16 (&s)[G], const float (&mxl)[G], bool first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const float mx = fmaxf(mxl[g], __shfl_xor(mxl[g], 32));
+            float alpha;
+            if constexpr (OFS) {
+                float m_new = m_run[g] + (first ? mx : fmaxf(mx, 0.f));
+                m_new = (float)(f16)fminf(fmaxf(m_new, -30000.f), 30000.f);
+                const float up = m_new - m_run[g];
+                alpha = first ? 0.f : fast_exp2(-up);
+                m_run[g] = m_new;
+                s[g] -= up;
+                const f16 nr = (f16)(-m_new);
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    if (ks == (d >> 4) && hl == ((d >> 3) & 1)) qf[g][ks][0] = nr;
+            } else {
+                const float m_new = fmaxf(m_run[g], mx * c);
+                alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run[g] - m_new);
+                m_run[g] = m_new;
+                nm[g] = m_new == -INFINITY ? 0.f : -m_new;
+                thr[g] = (m_new + kRescaleLog2) * inv_c;
+            }
+#pragma unroll
+            for (int t = 0; t < MTD; ++t) o[g][t] *= alpha;
+            l_run[g] *= alpha;
+        }
+    };
+
+    // One 32-key sub-tile: softmax and PV of cur, with the next sub-tile's QK in front of
+    // them, whose scores nxt are then checked against the references.  V: this sub-tile's rows;
+    // kn: the K rows of the sub-tile after the next; kv: valid keys of the next.
+    auto stage = [&](auto full, floatx16 (&cur)[G], floatx16 (&nxt)[G], const f16* vt, const f16* kn, int kv) __attribute__((always_inline)) {
+        half8 vf[2][MTD], pf[G][2];
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int t = 0; t < MTD; ++t) vf[st][t] = vt_frag<true>(vt, VSTR, t, st * 16, lrow, lk, 0);
+        qk(nxt);
+        load_kf(kn);
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float x = cur[g][st * 8 + i];
+                    const float p = fast_exp2(OFS ? x : __builtin_fmaf(x, c, nm[g]));
+                    if (!LSUM) l_run[g] += p;
+                    pf[g][st][i] = (f16)p;
+                }
+            }
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int t = 0; t < MTD; ++t) o[g][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[st][t], pf[g][st], o[g][t], 0, 0, 0);
+        if constexpr (!full.value) mask(nxt, kv);
+        float mx[G];
+        lane_max(nxt, mx);
+        bool up = false;
+#pragma unroll
+        for (int g = 0; g < G; ++g) up |= mx[g] > (OFS ? kRescaleLog2 : thr[g]);
+        if constexpr (full.value) {
+#pragma unroll
+            for (int i = 0; i < KS * G; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);              // MFMA
+                if (i * 2 < 4 * MTD) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // LDS reads
+                __builtin_amdgcn_sched_group_barrier(0x002, OFS ? 2 : 6, 0);    // VALU
+                __builtin_amdgcn_sched_group_barrier(0x400, 24 / (KS * G), 0);  // exp
+            }
+#pragma unroll
+            for (int i = 0; i < 4 * MTD; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (i < KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                if (i < 4) __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+            }
+        }
+        if (__ballot(up)) rebase(nxt, mx, false);
+    };
+
+    floatx16 sa[G], sb[G];
+    load_kf(Ks + klo);
+    qk(sa);
+    load_kf(Ks + 32 * KSTR + klo);
+    mask(sa, a.Sk);
+    {
+        float mx[G];
+        lane_max(sa, mx);
+        rebase(sa, mx, true);
+    }
+    int b0 = 0, b1 = 1, b2 = 2, left = a.Sk;  // ring buffers of tiles it, it + 1, it + 2; keys from tile it on
+    auto tile = [&](auto full) __attribute__((always_inline)) {
+        // tile it + 2 takes the buffer of tile it - 1, which every wave left at the last barrier
+        store_kv(b2);
+        load_kv();
+        const f16* vt = Vs + b0 * VTILE + vlo;
+        const f16* kn = Ks + b1 * KTILE + klo;
+        __builtin_amdgcn_sched_barrier(0);
+        stage(full, sa, sb, vt, kn, left - 32);
+        // (past the last tile: no keys, nothing to rebase to)
+        stage(full, sb, sa, vt + 32 * VSTR, kn + 32 * KSTR, left - 64);
+        left -= KT;
+        const int t = b0;
+        b0 = b1;
+        b1 = b2;
+        b2 = t;
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS stores and reads are done
+        __builtin_amdgcn_s_barrier();
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    };
+#pragma nounroll
+    while (left >= KT + 32) tile(std::true_type{});
+#pragma nounroll
+    while (left > 0) tile(std::false_type{});
+
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const float inv = 1.0f / row_sum<MTD, LSUM>(o[g], l_run[g], lrow);
+        const int q = q0 + g * 32 + lrow;
+        if (q >= a.Sq) continue;
+        f16* op = a.o + ((int64_t)b * a.Sq + q) * a.ldo + (int64_t)h * d;
+#pragma unroll
+        for (int t = 0; t < MTD; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; e += 4) {
+                const int dim = t * 32 + (e >> 2) * 8 + hl * 4;
+                if (dim >= d) continue;
+                uint2 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ((f16*)&v)[i] = (f16)(o[g][t][e + i] * inv);
+                *(uint2*)(op + dim) = v;
+            }
+    }
+}
+
 // ----------------------------------------------------------------- key-split kernel
 
 static constexpr int KTS = 32;         // keys per step
@@ -727,7 +1010,7 @@ static int resident_blocks(Kern kern, int threads) {
 struct AttnPlan {
     bool shared;
     int nw, ns;
-    bool kt128, ofs, spl;
+    bool kt128, ofs, spl, wide;
     dim3 grid;
 };
 
@@ -748,6 +1031,18 @@ static AttnPlan attn_plan(const AttnArgs& a) {
         p.shared = true;
         p.nw = (a.d > 48 && a.d <= 128 && ((a.Sq + 127) / 128) * bh < 512) ? 8 : 4;
         p.grid = dim3((a.Sq + p.nw * 32 - 1) / (p.nw * 32), a.heads, a.B);
+        // 64 queries per wave for heads of 33..64 where their 256-query blocks cover more than
+        // half of the CUs (144 blocks and up) and leave no short second round (257..320 of 256
+        // CUs).  Time against the narrow tiles', d 40 / d 64: 128 blocks 0.9-1.1 / 0.8-1.0,
+        // 144 to 256 0.78-0.87 / 0.81-0.98, 257 to 320 1.02-1.08 / 0.78-1.05, above 0.45-0.97 /
+        // 0.7-0.9.  Heads up to 32 have half the PV work per exp and lose (0.9-1.4).
+        const long nwide = (long)((a.Sq + 255) / 256) * bh;
+        if ((KS == 3 || KS == 4) && nwide >= 144 && (nwide <= 256 || nwide > 320)) {
+            p.wide = true;
+            p.ofs = a.q_log2 && a.d < KS * 16;
+            p.grid = dim3((a.Sq + 255) / 256, a.heads, a.B);
+            return p;
+        }
         // 128-key tiles for heads <= 48 when every block is resident at once (two per CU):
         // d40 at 4096 tokens, B=2, 0.44 ms per forward against 0.46 with 64-key tiles;
         // on larger grids they lose (0.24 ms more at 9216 tokens, 0.31 ms at B=16)
@@ -796,6 +1091,16 @@ static void launch_cfg(const AttnArgs& a0, hipStream_t s) {
     const double flops = 4.0 * bh * a.Sq * a.Sk * a.d;
     const double bytes = 2.0 * bh * a.d * (2.0 * a.Sq + 2.0 * a.Sk);
     char name[48];
+    if constexpr (KS == 3 || KS == 4) {
+        if (p.wide) {
+            snprintf(name, sizeof name, "attn_wide_kernel<%d,%d,%d,%d>", KS, MTD, (int)LSUM, (int)p.ofs);
+            launch_timed(name, flops, bytes, [&] {
+                if (p.ofs) SDU_LAUNCH((attn_wide_kernel<KS, MTD, LSUM, true>), p.grid, dim3(256), 0, s, a);
+                else SDU_LAUNCH((attn_wide_kernel<KS, MTD, LSUM, false>), p.grid, dim3(256), 0, s, a);
+            });
+            return;
+        }
+    }
     if (p.shared) {
         const bool spl = p.spl && a.ws;
         const bool trv = kTRV && !p.kt128;

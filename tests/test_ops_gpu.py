@@ -579,6 +579,19 @@ def test_attention_q_log2_reference_moves(op_engine, B):
     assert np.abs(got - ref).max() < 2e-2
 
 
+@pytest.mark.parametrize("B,heads,Sq,Sk,d", [
+    (18, 8, 225, 129, 40),   # 144 query blocks, the fewest; one key past the second tile
+    (18, 8, 256, 160, 48),   # no spare dimension for the reference; an odd number of 32-key steps
+    (32, 8, 257, 191, 56),   # a query block of one; a key short of a tile
+    (19, 8, 250, 193, 64),   # row sums outside the MFMA
+    (41, 8, 290, 256, 40),   # whole tiles; two rounds of blocks
+])
+def test_attention_wide(op_engine, B, heads, Sq, Sk, d):
+    """Edges of the 64-queries-per-wave kernel's query blocks and key steps, with either form of the scale."""
+    test_attention(op_engine, B, heads, Sq, Sk, d)
+    test_attention_q_log2(op_engine, B, heads, Sq, Sk, d)
+
+
 # ------------------------------------------------------------------ elementwise
 
 
