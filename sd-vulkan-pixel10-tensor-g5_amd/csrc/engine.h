@@ -160,7 +160,9 @@ struct Ctx {
     // op-level tensors and per-shape forward state
     std::vector<FwdState*> fwd;  // owned; freed by free_fwd_states (LRU-capped)
     uint64_t use_clock = 0;
-    float* op_ws = nullptr;     // scratch for op-level calls
+    // scratch for op-level calls: the split-K / attention counters at its head (gemm_counter_bytes,
+    // cleared when it is allocated and left zero by every launch), then the op's own
+    float* op_ws = nullptr;
     size_t op_ws_bytes = 0;
 
     // auxiliary networks (created on demand by sdu_taesd_init / sdu_clip_init)
@@ -205,7 +207,7 @@ int load_weight_file(Ctx& c, const WeightRec& r, const std::string& dir);
 // Allocate an auxiliary network's pool for its registered tensors and place them.
 int aux_alloc(Ctx& c, AuxNet& n, size_t extra_bytes);
 void aux_free(AuxNet* n);
-int ensure_op_ws(Ctx& c, size_t bytes);
+int ensure_op_ws(Ctx& c, size_t bytes);  // bytes >= gemm_counter_bytes(), counters included
 int set_err(Ctx* c, int code, const std::string& msg);
 
 // taesd.cpp: latent [B, 4, H, W] fp32 -> image [B, 3, 8H, 8W] fp32 in about [-1, 1]

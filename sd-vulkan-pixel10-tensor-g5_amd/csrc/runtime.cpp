@@ -468,6 +468,11 @@ int ensure_op_ws(Ctx& c, size_t bytes) {
         c.op_ws_bytes = 0;
     }
     if (hipMalloc(&c.op_ws, bytes) != hipSuccess) return set_err(&c, SDU_ERR_OOM, "op workspace allocation failed");
+    if (zero_launch(c.op_ws, gemm_counter_bytes(), c.stream) != hipSuccess) {
+        hipFree(c.op_ws);
+        c.op_ws = nullptr;
+        return set_err(&c, SDU_ERR_HIP, "op workspace clear failed");
+    }
     c.op_ws_bytes = bytes;
     return SDU_OK;
 }

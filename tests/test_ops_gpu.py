@@ -592,6 +592,17 @@ def test_attention_wide(op_engine, B, heads, Sq, Sk, d):
     test_attention_q_log2(op_engine, B, heads, Sq, Sk, d)
 
 
+def test_split_ops_share_scratch(op_engine):
+    """Split launches of each kind between each other and other users of the scratch: every launch
+    leaves the arrival counters at its head zero and no op's own scratch reaches them."""
+    for _ in range(2):
+        test_matmul(op_engine, 70, 72, 2048, 0, True, True, False, False)
+        test_groupnorm(op_engine, 2, 64, 64, 640, 320, True)
+        test_attention_q_log2(op_engine, 5, 8, 1800, 300, 56)  # keys split in two
+        test_conv_groupnorm_epilogue_stats(op_engine, 2, 8, 8, 1280, 1280, 0.0, True, False, True)
+        test_conv_patch_tiles(op_engine, 2, 8, 8, 1280, 1280, False, True)
+
+
 # ------------------------------------------------------------------ elementwise
 
 
