@@ -804,88 +804,99 @@ void gemm_kernel(GemmArgs a) {
     }
 }
 
-// 3x3 conv (pad 1, stride 1, no upsample) with at most 8 output channels (the UNet's
-// conv_out, 320 -> 4): an MFMA tile would be 64 columns wide for 4, and 64 such tiles
-// cannot fill the chip.  One thread per (pixel, K slice), 16 pixels x 16 slices per
-// block: slice s takes the 8-channel chunks j = s, s + 16, ... of the pixel's 9 Cin / 8
-// (tap-major, as W's K index) with fp16 dot products into fp32, the weights staged
-// in LDS (dynamic, CO * 9 * Cin * 2 bytes); the 16 slices of a pixel are consecutive
-// lanes, added by shuffles, and the first runs the common epilogue.  Loads go in
-// batches of 12 chunks (two batches at Cin = 320), all issued before any is used.  A
-// block takes 16-pixel groups g, g + gridDim.x, ... (at most kNarrowBlocks blocks), so on
-// large images (the VAE's 512x512 conv_out) the staged weights serve many groups.
-constexpr int kNarrowPix = 16, kNarrowSlices = 16, kNarrowBatch = 12, kNarrowBlocks = 2048;
-template <int CO>
+// 3x3 conv (pad 1, stride 1, no upsample) with at most 8 output channels (the UNet's and the
+// decoders' conv_out).  The taps go into the matrix product's columns: row (tap, co) of a
+// [9 CO][Cin] weight times the pixels of a T x T tile and its border, so every pixel is read once,
+// straight into its MFMA operand, and the product is formed for 9 CO (36 of 48) columns instead
+// of nine times for 16; then each output pixel adds its nine taps' products from LDS.
+// Bound by the input's bytes and the border's re-reads on large images (512 x 512 x 64 -> 3: 14 us,
+// 34 MB at 2.3 TB/s), by the latency of the K steps on small ones.  Against one thread per (pixel,
+// K slice) with fp16 dot products (us): 512 x 512 x 64 -> 3 80 -> 14, 512 x 512 x 128 -> 3 103 -> 23,
+// 16 x 64 x 64 x 320 -> 4 58 -> 16, 2 x 64 x 64 x 320 -> 4 12.5 -> 7.8, 512 x 512 x 64 -> 8 118 -> 38,
+// 16 x 16 x 448 -> 8 19 -> 12.5.
+template <int CO, int T>
 __global__ __launch_bounds__(256) void conv3_narrow_kernel(GemmArgs a) {
     if (a.c_ind) a.C = *a.c_ind;
-    typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-    extern __shared__ uint4 wsm[];  // [CO][nchunk]
-    const int cpt = a.Cin / 8, nchunk = 9 * cpt;
-    {
-        // CO * nchunk <= 4096 chunks (narrow_conv): at most 16 per thread, loads first
-        constexpr int SMAX = 4096 / (kNarrowPix * kNarrowSlices);
-        uint4 wv[SMAX];
+    constexpr int PW = T + 2, NPX = PW * PW, MT = (NPX + 15) / 16, MW = (MT + 3) / 4, NJ = (9 * CO + 15) / 16;
+    constexpr int TS = CO == 4 ? 36 : 76;  // floats per pixel: an odd number of 16-byte chunks
+    __shared__ __attribute__((aligned(16))) float prod[MT * 16 * TS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lq = lane >> 4, lr = lane & 15;
+    const int nbx = (a.Wo + T - 1) / T, nby = (a.Ho + T - 1) / T, spi = nbx * nby;
+    const int bid = xcd_block(gridDim.x, blockIdx.x), b = bid / spi, r0 = bid - b * spi;
+    const int y0 = r0 / nbx * T, x0 = (r0 - r0 / nbx * nbx) * T;
+    constexpr uint32_t kOOB = 0x80000000u;
+    // byte offsets of the lane's pixel of each of the wave's 16-pixel tiles, and of its weight row
+    // (tap, co) of each 16 columns; pixels outside the image and rows past 9 CO read zeros
+    uint32_t vp[MW], vw[NJ];
 #pragma unroll
-        for (int u = 0; u < SMAX; ++u) {
-            const int i = threadIdx.x + u * kNarrowPix * kNarrowSlices, co = i / nchunk, j = i - co * nchunk;
-            wv[u] = make_uint4(0, 0, 0, 0);
-            if (i < CO * nchunk && co < a.N) wv[u] = *(const uint4*)(a.Wt + (int64_t)co * a.K + j * 8);
-        }
-#pragma unroll
-        for (int u = 0; u < SMAX; ++u) {
-            const int i = threadIdx.x + u * kNarrowPix * kNarrowSlices;
-            if (i < CO * nchunk) wsm[i] = wv[u];
-        }
+    for (int i = 0; i < MW; ++i) {
+        const int r = (wave + 4 * i) * 16 + lr, py = r / PW, y = y0 + py - 1, x = x0 + (r - py * PW) - 1;
+        vp[i] = r < NPX && y >= 0 && y < a.Hin && x >= 0 && x < a.Win ? (uint32_t)(((b * a.Hin + y) * a.Win + x) * a.Cin * 2) : kOOB;
     }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int n = j * 16 + lr, tap = n / CO, co = n % CO;
+        vw[j] = tap < 9 && co < a.N ? (uint32_t)((co * a.K + tap * a.Cin) * 2) : kOOB;
+    }
+    const __amdgpu_buffer_rsrc_t rsA =
+        __builtin_amdgcn_make_buffer_rsrc((void*)a.A, (short)0, a.Bn * a.Hin * a.Win * a.Cin * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsW = __builtin_amdgcn_make_buffer_rsrc((void*)a.Wt, (short)0, a.N * a.K * 2, 0x00020000);
+    const int nch = a.Cin >> 3;
+    struct Frag {
+        half8 p[MW], w[NJ];
+    };
+    auto load = [&](Frag& f, int ks) __attribute__((always_inline)) {
+        const int kc = ks * 4 + lq;  // 8-channel chunk
+        const uint32_t ko = kc * 16, off = kc < nch ? 0u : kOOB;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            f.w[j] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rsW, (vw[j] + ko) | off, 0, 0));
+#pragma unroll
+        for (int i = 0; i < MW; ++i)
+            f.p[i] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rsA, (vp[i] + ko) | off, 0, 0));
+    };
+    floatx4 acc[MW][NJ];
+#pragma unroll
+    for (int i = 0; i < MW; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{};
+    auto mfma = [&](const Frag& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MW; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.w[j], f.p[i], acc[i][j], 0, 0, 0);
+    };
+    Frag f0, f1;
+    load(f0, 0);
+#pragma nounroll
+    for (int ks = 0; ks * 4 < nch; ks += 2) {  // (steps past the last one multiply zeros)
+        load(f1, ks + 1);
+        mfma(f0);
+        load(f0, ks + 2);
+        mfma(f1);
+    }
+#pragma unroll
+    for (int i = 0; i < MW; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int mt = wave + 4 * i, n = j * 16 + lq * 4;
+            if (mt < MT && n < 9 * CO) *(floatx4*)&prod[(mt * 16 + lr) * TS + n] = acc[i][j];
+        }
     __syncthreads();
-    const int tid = threadIdx.x, sl = tid % kNarrowSlices;
-    const int ngroups = (a.M + kNarrowPix - 1) / kNarrowPix;
-    for (int grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
-        const int p = grp * kNarrowPix + tid / kNarrowSlices;
-        const int m = min(p, a.M - 1);
-        const int hw = a.Ho * a.Wo, bb = m / hw, r = m - bb * hw, oy = r / a.Wo, ox = r - oy * a.Wo;
-        float acc[CO];
+    for (int q = tid; q < T * T * (CO / 4); q += 256) {
+        const int p = q % (T * T), c4 = q / (T * T) * 4, py = p / T, px = p % T, y = y0 + py, x = x0 + px;
+        if (y >= a.Ho || x >= a.Wo) continue;
+        floatx4 v = floatx4{};
 #pragma unroll
-        for (int co = 0; co < CO; ++co) acc[co] = 0.f;
-        // chunks in batches: every load of a batch issued before any is used
-        for (int j0 = sl; j0 < nchunk; j0 += kNarrowSlices * kNarrowBatch) {
-            uint4 x[kNarrowBatch];
+        for (int tap = 0; tap < 9; ++tap)
+            v += *(const floatx4*)&prod[((py + tap / 3) * PW + px + tap % 3) * TS + tap * CO + c4];
+        const int m = (b * a.Ho + y) * a.Wo + x;
 #pragma unroll
-            for (int u = 0; u < kNarrowBatch; ++u) {
-                const int j = j0 + u * kNarrowSlices;
-                const int tap = j / cpt, c8 = j - tap * cpt;
-                const int iy = oy + tap / 3 - 1, ix = ox + tap % 3 - 1;
-                x[u] = make_uint4(0, 0, 0, 0);
-                if (j < nchunk && iy >= 0 && iy < a.Hin && ix >= 0 && ix < a.Win)
-                    x[u] = *(const uint4*)(a.A + (((int64_t)bb * a.Hin + iy) * a.Win + ix) * a.Cin + c8 * 8);
-            }
-#pragma unroll
-            for (int u = 0; u < kNarrowBatch; ++u) {
-                const int j = j0 + u * kNarrowSlices;
-                if (j >= nchunk) break;
-                const half2v* xh = (const half2v*)&x[u];
-#pragma unroll
-                for (int co = 0; co < CO; ++co) {
-                    const uint4 w = wsm[co * nchunk + j];
-                    const half2v* wh = (const half2v*)&w;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) acc[co] = __builtin_amdgcn_fdot2(xh[q], wh[q], acc[co], false);
-                }
-            }
-        }
-#pragma unroll
-        for (int co = 0; co < CO; ++co)
-#pragma unroll
-            for (int off = 1; off < kNarrowSlices; off <<= 1) acc[co] += __shfl_xor(acc[co], off);
-        if (sl == 0 && p < a.M) {
-#pragma unroll
-            for (int co = 0; co < CO; ++co)
-                if (co < a.N) epi_store(a, p, co, acc[co], 0.f, co);
-        }
+        for (int e = 0; e < 4; ++e)
+            if (c4 + e < a.N) epi_store(a, m, c4 + e, v[e], 0.f, c4 + e);
     }
 }
 
-// The narrow conv takes a 3x3 conv when its weights (up to 8 outputs) fit 64 KB of LDS.
 static bool narrow_conv(const GemmArgs& a) {
     return a.amode == A_CONV3 && a.N <= 8 && a.stride == 1 && !a.upsample && !a.A2 && !a.stats && !a.geglu &&
            !a.row_part && a.Cin % 8 == 0 && 8 * 9 * (a.Cin / 8) <= 4096 && a.M > 0;
@@ -942,6 +953,14 @@ const char* const kNames[kNumGemm][2] = {{"gemm_kernel<256,128,4,2,64,2,0,32>", 
                                         {"gemm_kernel<64,160,2,2,64,2,0,16>", "gemm_kernel<64,160,2,2,64,2,1,16>"}};
 
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// 16 x 16 pixel tiles (less border) where they give every CU one
+int narrow_tile(const GemmArgs& a) {
+    return a.N <= 4 && (int64_t)a.Bn * ceil_div(a.Ho, 16) * ceil_div(a.Wo, 16) >= 256 ? 16 : 8;
+}
+const char* narrow_name(const GemmArgs& a) {
+    return a.N > 4 ? "conv3_narrow_kernel<8,8>" : narrow_tile(a) == 16 ? "conv3_narrow_kernel<4,16>" : "conv3_narrow_kernel<4,8>";
+}
 
 // In-kernel split-K sum: tile counters at the head of the workspace (one per tile).
 constexpr int kMaxSplitTiles = 16384;
@@ -1031,7 +1050,7 @@ void plan(const GemmArgs& a, int& ci, int& splits, int& kps, bool& fix) {
 bool gemm_stats_supported(int hw) { return stats_tile_ok(128, hw); }
 
 std::string gemm_kernel_name(const GemmArgs& a) {
-    if (narrow_conv(a)) return a.N <= 4 ? "conv3_narrow_kernel<4>" : "conv3_narrow_kernel<8>";
+    if (narrow_conv(a)) return narrow_name(a);
     int ci, splits, kps;
     bool fix;
     plan(a, ci, splits, kps, fix);
@@ -1066,15 +1085,15 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
             return hipErrorInvalidValue;
         a.splits = 1;
         a.partial = nullptr;
-        const int co = a.N <= 4 ? 4 : 8;
-        const size_t lds = (size_t)co * 9 * a.Cin * 2;
-        const dim3 grid(std::min((a.M + kNarrowPix - 1) / kNarrowPix, kNarrowBlocks));
+        const int t = narrow_tile(a);
+        const dim3 grid(a.Bn * ceil_div(a.Ho, t) * ceil_div(a.Wo, t)), blk(256);
         const double flops = 2.0 * a.M * a.N * a.K;
         const double bytes = 2.0 * a.Bn * a.Hin * a.Win * a.Cin + 2.0 * a.N * a.K +
                              (double)a.M * a.N * (a.out_mode == OUT_F16 ? 2.0 : 4.0) + (a.res ? 2.0 * a.M * a.N : 0.0);
-        launch_timed(co == 4 ? "conv3_narrow_kernel<4>" : "conv3_narrow_kernel<8>", flops, bytes, [&] {
-            if (co == 4) SDU_LAUNCH(conv3_narrow_kernel<4>, grid, dim3(kNarrowPix * kNarrowSlices), lds, s, a);
-            else SDU_LAUNCH(conv3_narrow_kernel<8>, grid, dim3(kNarrowPix * kNarrowSlices), lds, s, a);
+        launch_timed(narrow_name(a), flops, bytes, [&] {
+            if (a.N > 4) SDU_LAUNCH((conv3_narrow_kernel<8, 8>), grid, blk, 0, s, a);
+            else if (t == 16) SDU_LAUNCH((conv3_narrow_kernel<4, 16>), grid, blk, 0, s, a);
+            else SDU_LAUNCH((conv3_narrow_kernel<4, 8>), grid, blk, 0, s, a);
         });
         return hipGetLastError();
     }

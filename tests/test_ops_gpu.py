@@ -391,6 +391,19 @@ def test_matmul_inplace_residual(op_engine, M, N, K):
     assert np.abs(got - ref).max() < 3e-2
 
 
+@pytest.mark.parametrize("B,H,W,Ci,Co,temb,res", [
+    (1, 5, 3, 8, 1, True, True),         # one tile, an eighth of a K step
+    (2, 17, 9, 72, 3, False, True),      # a K tail of one 8-channel chunk; ragged tiles
+    (3, 9, 16, 320, 4, True, False),     # ten K steps
+    (2, 11, 8, 96, 5, True, True),       # 5..8 outputs; an odd number of K steps
+    (1, 16, 24, 448, 8, False, False),   # the most channels the form takes
+    (1, 257, 255, 64, 3, False, False),  # 16 x 16 tiles, a row past the last whole one, a column short of it
+])
+def test_conv_narrow_tiles(op_engine, B, H, W, Ci, Co, temb, res):
+    """Edges of the narrow-output conv's tiles and K steps."""
+    test_conv2d(op_engine, B, H, W, Ci, Co, 3, 1, False, temb, res)
+
+
 def test_conv2d_inplace_residual_and_overlap_errors(op_engine):
     """A conv's residual may be its output; an output over the conv's or a matmul's own
     operands is an argument error (other tiles still read what it would overwrite)."""
