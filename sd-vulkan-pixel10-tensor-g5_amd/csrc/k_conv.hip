@@ -79,7 +79,8 @@ void conv3_patch_kernel(GemmArgs a) {
     constexpr int PATCH = PQ * 1024, BST = BQ * 1024;                        // bytes
     constexpr int SMEM = 2 * PATCH + NS * BST;
     // patch DMA of the next chunk: APT instructions in each of the first taps, none in the last one
-    constexpr int APT = (AI + NTAP - 3) / (NTAP - 2), LASTA = (AI - 1) / APT;
+    // (a ring of all taps: before the first weights of that chunk are asked for)
+    constexpr int APT = NS == NTAP ? (NTAP == 9 ? AI : (AI + 1) / 2) : (AI + NTAP - 3) / (NTAP - 2), LASTA = (AI - 1) / APT;
     static_assert(WTM % 32 == 0 && WTN % 16 == 0 && NTAP % NS == 0 && LASTA <= NTAP - NS + (NTAP == 4) && SMEM <= 160 * 1024, "tile");
     static_assert(SPX % WTM == 0 || (TW == 8 && WTM % 64 == 0), "wave rows");
     __shared__ __attribute__((aligned(1024))) char smem[SMEM];
@@ -494,12 +495,16 @@ static const PatchCfg kPatch[kNumPatch] = {
     {16, 1, 128, 512, {"conv3_patch_kernel<16,1,128,4,2,9>", "conv3_patch_kernel<16,1,128,4,2,4>"}},
     {16, 1, 160, 512, {"conv3_patch_kernel<16,1,160,4,2,9>", ""}},
     {8, 2, 80, 256, {"conv3_patch_kernel<8,2,80,4,1,9>", "conv3_patch_kernel<8,2,80,4,1,4>"}},
-    {8, 2, 64, 256, {"conv3_patch_kernel<8,2,64,4,1,9>", "conv3_patch_kernel<8,2,64,4,1,4>"}}};
+    {8, 2, 64, 256, {"conv3_patch_kernel<8,2,64,4,1,9>", "conv3_patch_kernel<8,2,64,4,1,4>"}},
+    {8, 2, 64, 256, {"conv3_patch_kernel<8,2,64,4,1,9,9>", ""}},
+    {8, 1, 64, 256, {"conv3_patch_kernel<8,1,64,2,2,9,9>", ""}},
+    {8, 1, 32, 128, {"conv3_patch_kernel<8,1,32,2,1,9,9>", ""}}};
 
 const char* conv_patch_name(int cfg, bool subpix) { return kPatch[cfg].name[subpix]; }
 
-// (four 160-wide weight tiles do not fit the LDS)
-bool conv_patch_subpix(int cfg) { return cfg != 1; }
+// (four 160-wide weight tiles do not fit the LDS; the shapes with a ring of all nine taps' weights
+// have no four-tap form)
+bool conv_patch_subpix(int cfg) { return cfg != 1 && cfg < 4; }
 
 int conv_patch_tiles_m(int cfg, const GemmArgs& a) {
     const PatchCfg& p = kPatch[cfg];
@@ -517,6 +522,9 @@ void conv_patch_launch(int cfg, const GemmArgs& a, hipStream_t s) {
         case 4: SDU_LAUNCH((conv3_patch_kernel<8, 2, 80, 4, 1, 9, 3, 2>), grid, blk, 0, s, a); break;
         case 5: SDU_LAUNCH((conv3_patch_kernel<8, 2, 80, 4, 1, 4, 4, 1>), grid, blk, 0, s, a); break;
         case 6: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 9, 3, 2>), grid, blk, 0, s, a); break;
+        case 8: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 9, 9, 1>), grid, blk, 0, s, a); break;
+        case 10: SDU_LAUNCH((conv3_patch_kernel<8, 1, 64, 2, 2, 9, 9, 1>), grid, blk, 0, s, a); break;
+        case 12: SDU_LAUNCH((conv3_patch_kernel<8, 1, 32, 2, 1, 9, 9, 1>), grid, blk, 0, s, a); break;
         case 7: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 4, 4, 1>), grid, blk, 0, s, a); break;
     }
 }

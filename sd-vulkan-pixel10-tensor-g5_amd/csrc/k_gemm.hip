@@ -917,18 +917,24 @@ struct Cfg {
 // 2: 128x64,  8 waves of 32x32, BK 64, 3-stage ring (72 KB: two per CU, 4 waves per SIMD)
 // 3: 64x160,  4 waves of 32x80 (16x16x32 MFMAs), BK 64, 2-stage ring (56 KB: two per CU)
 // 4 ..: the patch-resident conv kernel's shapes (k_conv.hip): 16x16 pixels x 128 or 160
-// channels (8 waves, one block per CU), two 8x8 sub-tiles x 80 or 64 channels (4 waves, two)
+// channels (8 waves, one block per CU), two 8x8 sub-tiles x 80 or 64 channels (4 waves, two);
+// with all nine taps' weights in the ring, for launches of few blocks: two sub-tiles x 64
+// (4 waves, one), one sub-tile x 64 (4 waves, one) or 32 (2 waves, two)
 // Rates and fixed costs of 0..3 from dense GEMMs that give every CU one or two blocks, at
 // K = 512 and 4096 (the difference gives the rate, the rest the fixed cost).  The 64x160
 // tile covers N = 320 with no padded column and M = 8192 with 256 tiles, so it fills the
 // chip where 128-row tiles leave a quarter of the CUs idle, but its own rate is lower (4
 // waves, 46 FLOP per operand byte against 64).  The implicit-conv A (a tap gather per row)
 // costs the 64-column tile about 20% of its rate.
-// 4 ..: fitted to 1700 launches over 44 conv shapes (8x8 to 512x512 pixels, 64 to 2560
-// channels, batches 1 to 16, ragged sizes; every shape and split count timed): the planner's
-// choice is within 3% of the best of them on all but two (4%), and always a shape of
-// this kernel, so the convs it can take are planned among these alone.
-// 8 ..: gemm_dense_kernel's shapes (k_dense.hip): 256x128 (8 waves, one block per CU),
+// 4 ..: fitted to 3400 launches over 48 conv shapes (8x8 to 512x512 pixels, 64 to 2560
+// channels, batches 1 to 16, ragged sizes; every shape and split count), those of few blocks
+// timed with operands in the caches and out of them and weighed alike: the planner's choice is
+// within 5% of the best of them on all but five (8%), and always a shape of this kernel, so
+// the convs it can take are planned among these alone.  The deep rings gain from cold weights
+// (64x64x512 33 -> 27 us, 2x36x28x640 38 -> 28), the small tiles where a launch is one
+// short round (64x64x64 9.4 -> 7.3 warm, 11.6 -> 7.2 cold); two sub-tiles x 80 with all taps
+// gained 6-10% cold and lost as much warm.
+// 11 ..: gemm_dense_kernel's shapes (k_dense.hip): 256x128 (8 waves, one block per CU),
 // 128x128, 128x64 (4 waves, two) and 64x64 (4 waves, three), fitted the same way to 2400
 // launches over 50 dense shapes (1 to 65536 rows, K 64 to 6400).
 enum Kind { K_GEMM = 0, K_PATCH = 1, K_DENSE = 2 };
@@ -937,10 +943,13 @@ const Cfg kCfgs[kNumCfg] = {{256, 128, 1, 3.5e12, 3.5e12, 4.5e-6, 1, 1.0, K_GEMM
                             {128, 128, 2, 2.76e12, 3.9e12, 3.0e-6, 1, 1.0, K_GEMM, 1, 0.9e-6},
                             {128, 64, 2, 2.23e12, 3.03e12, 2.5e-6, 2, 0.8, K_GEMM, 2, 0.9e-6},
                             {64, 160, 2, 2.0e12, 3.4e12, 6.0e-6, 2, 0.9, K_GEMM, 3, 0.9e-6},
-                            {256, 128, 1, 6.8e12, 6.8e12, 8.2e-6, 1, 1.0, K_PATCH, 0, 1.0e-6},
-                            {256, 160, 1, 6.0e12, 6.0e12, 8.8e-6, 1, 1.0, K_PATCH, 1, 1.2e-6},
-                            {128, 80, 2, 5.07e12, 5.2e12, 4.75e-6, 1, 1.0, K_PATCH, 2, 0.39e-6},
-                            {128, 64, 2, 4.63e12, 5.08e12, 4.0e-6, 1, 1.0, K_PATCH, 3, 0.33e-6},
+                            {256, 128, 1, 6.61e12, 6.61e12, 8.1e-6, 1, 1.0, K_PATCH, 0, 1.24e-6},
+                            {256, 160, 1, 5.93e12, 5.93e12, 8.6e-6, 1, 1.0, K_PATCH, 1, 1.73e-6},
+                            {128, 80, 2, 4.36e12, 5.06e12, 5.5e-6, 1, 1.0, K_PATCH, 2, 0.81e-6},
+                            {128, 64, 2, 4.05e12, 5.5e12, 5.2e-6, 1, 1.0, K_PATCH, 3, 0.5e-6},
+                            {128, 64, 1, 4.86e12, 4.86e12, 7.1e-6, 1, 1.0, K_PATCH, 4, 0.12e-6},
+                            {64, 64, 1, 3.93e12, 3.93e12, 5.4e-6, 1, 1.0, K_PATCH, 5, 0.08e-6},
+                            {64, 32, 2, 2.08e12, 3.82e12, 5.0e-6, 1, 1.0, K_PATCH, 6, 0.11e-6},
                             {256, 128, 1, 5.5e12, 5.5e12, 4.6e-6, 1, 1.0, K_DENSE, 0, 1.07e-6},
                             {128, 128, 2, 3.76e12, 4.5e12, 3.1e-6, 1, 1.0, K_DENSE, 1, 0.97e-6},
                             {128, 64, 2, 3.57e12, 3.8e12, 2.2e-6, 1, 1.0, K_DENSE, 2, 0.68e-6},
@@ -971,7 +980,7 @@ constexpr size_t kCounterBytes = kMaxSplitTiles * sizeof(unsigned);
 struct SplitCost {
     double rate, fix, red;
 };  // by Kind
-constexpr SplitCost kSplit[3] = {{20.0e12, 1.0e-6, 5.5e-6}, {38.0e12, 2.9e-6, 4.2e-6}, {12.0e12, 0.3e-6, 4.5e-6}};
+constexpr SplitCost kSplit[3] = {{20.0e12, 1.0e-6, 5.5e-6}, {38.0e12, 3.55e-6, 5.2e-6}, {12.0e12, 0.3e-6, 4.5e-6}};
 
 std::string cfg_name(int ci, const GemmArgs& a) {
     const Cfg& g = kCfgs[ci];

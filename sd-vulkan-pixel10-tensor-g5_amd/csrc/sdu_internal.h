@@ -167,7 +167,7 @@ hipError_t splitk_reduce_launch(const GemmArgs& a, double bytes, hipStream_t s);
 // The patch-resident 3x3 conv kernel (k_conv.hip): tile shape `cfg` of kNumPatch, for the
 // A_CONV3 GEMMs that gemm_launch sends there (stride 1, no upsample, Cin % 64 == 0, N % 8 ==
 // 0, fp16 or fp32 rows out, any splits).
-constexpr int kNumPatch = 4;
+constexpr int kNumPatch = 7;
 int conv_patch_tiles_m(int cfg, const GemmArgs& a);
 bool conv_patch_subpix(int cfg);  // the shape has a sub-pixel form
 const char* conv_patch_name(int cfg, bool subpix);

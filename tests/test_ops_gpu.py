@@ -366,6 +366,10 @@ def test_conv2d(op_engine, B, H, W, Ci, Co, k, stride, ups, temb, res):
     (1, 250, 243, 128, 128, True, False),  # 16x16 sub-tiles, both directions ragged
     (2, 8, 8, 1280, 1280, False, True),    # split K with the reduce launch
     (1, 16, 16, 704, 320, True, False),    # 11 chunks over uneven splits
+    (2, 36, 28, 640, 640, True, True),     # all taps' weights in the ring: 10 chunks
+    (1, 33, 39, 64, 72, False, True),      # one sub-tile x 32 columns, one chunk, ragged
+    (1, 128, 120, 64, 64, True, True),     # one sub-tile x 64 columns
+    (1, 16, 16, 1280, 1280, True, True),   # small tiles, split K
 ])
 def test_conv_patch_tiles(op_engine, B, H, W, Ci, Co, temb, res):
     """Edges of the patch-resident 3x3 kernel's tiles: 8x8 and 16x16 sub-tiles of ragged
