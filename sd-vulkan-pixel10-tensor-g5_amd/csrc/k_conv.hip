@@ -55,6 +55,11 @@ __device__ __forceinline__ void static_for(F&& f) {
 // empty resource so that every wait counts the same DMA, and the fragments of the next half
 // step are read during the MFMAs of this one (the block barrier comes in mid-step, after which
 // the next weight tile has landed and the oldest one may be overwritten).
+//
+// ONE: a conv of one 64-channel chunk without a tail or split: no second patch, so two 16x16 tiles
+// of 64 channels fit a CU and one's loads and epilogue run beside the other's taps
+// (512x512x64 -> 64 with residual 43 us -> 35, 110 MB at 3.1 TB/s; 300x400 22 -> 18; sub-pixel,
+// 256x256x64 to 512x512 50 -> 24).
 // DMA instructions a wave may have in flight at the barrier of tap t: those issued after the
 // step of the weights of step t + 1, i.e. NS - 2 weight tiles and the patch instructions of the
 // last NS - 2 taps (none of them before tap 0, see LASTA); after the last tap only what was
@@ -68,7 +73,7 @@ constexpr int dma_ahead(int t) {
     return t < NTAP - 1 || w < since_patch ? w : since_patch;
 }
 
-template <int TW, int NSUB, int NT, int WM, int WN, int NTAP, int NS, int WPE>
+template <int TW, int NSUB, int NT, int WM, int WN, int NTAP, int NS, int WPE, bool ONE = false>
 __global__ __launch_bounds__(WM* WN * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void conv3_patch_kernel(GemmArgs a) {
     constexpr int NW = WM * WN, NTH = NW * 64, SPX = TW * TW, MT = SPX * NSUB, WTM = MT / WM, WTN = NT / WN;
@@ -77,7 +82,7 @@ void conv3_patch_kernel(GemmArgs a) {
     constexpr int PQ = (NSUB * PPX * 8 + 63) / 64, AI = (PQ + NW - 1) / NW;  // 1 KB DMA instructions: patch, per wave
     constexpr int BQ = NT / 8, BI = (BQ + NW - 1) / NW;                      // weight tile, per wave
     constexpr int PATCH = PQ * 1024, BST = BQ * 1024;                        // bytes
-    constexpr int SMEM = 2 * PATCH + NS * BST;
+    constexpr int RING = (ONE ? 1 : 2) * PATCH, SMEM = RING + NS * BST;
     // patch DMA of the next chunk: APT instructions in each of the first taps, none in the last one
     // (a ring of all taps: before the first weights of that chunk are asked for)
     constexpr int APT = NS == NTAP ? (NTAP == 9 ? AI : (AI + 1) / 2) : (AI + NTAP - 3) / (NTAP - 2), LASTA = (AI - 1) / APT;
@@ -183,7 +188,7 @@ void conv3_patch_kernel(GemmArgs a) {
 #pragma unroll
         for (int i = 0; i < BI; ++i) {
             const int qi = i * NW + wave < BQ ? i * NW + wave : wave;
-            bdma(rs, voB[i], kw * 2, 2 * PATCH + st * BST + qi * 1024);
+            bdma(rs, voB[i], kw * 2, RING + st * BST + qi * 1024);
         }
     };
     // K offset of the weights d steps after the first step of unit u (d < NTAP), and whether
@@ -234,7 +239,7 @@ void conv3_patch_kernel(GemmArgs a) {
             oA[kx][0] = ((wrow / SPX * PW + y + oy0) * PW + px) * 128 + ((lq ^ sw) & 7) * 16;
             oA[kx][1] = oA[kx][0] ^ 64;
         }
-        oB[0] = 2 * PATCH + (wn * WTN + lr) * 128 + ((lq ^ (lr >> 1)) & 7) * 16;
+        oB[0] = RING + (wn * WTN + lr) * 128 + ((lq ^ (lr >> 1)) & 7) * 16;
         oB[1] = oB[0] ^ 64;
     }
     half8 af[2][FM], bf[2][FN];
@@ -292,17 +297,17 @@ void conv3_patch_kernel(GemmArgs a) {
                 mfma(0);
                 weave();
                 __builtin_amdgcn_sched_barrier(0);
-                wait_vmcnt_lgkm0<dma_ahead<NTAP, NS, BI, APT, AI>(tap)>();
+                wait_vmcnt_lgkm0<dma_ahead<NTAP, NS, BI, APT, ONE ? 0 : AI>(tap)>();
                 __builtin_amdgcn_s_barrier();
                 __atomic_signal_fence(__ATOMIC_SEQ_CST);
                 if constexpr (tap + NS < NTAP) issue_b(rsB, (tap + NS) * a.Cin + u * 64, tap % NS);
                 else issue_b_at(u + 1, tap + NS - NTAP, tap % NS);
 #pragma unroll
-                for (int i = tap * APT; i < (tap + 1) * APT && i < AI; ++i) issue_a(sn, i, pbuf ^ 1);
+                for (int i = tap * APT; !ONE && i < (tap + 1) * APT && i < AI; ++i) issue_a(sn, i, pbuf ^ 1);
                 if constexpr (tap + 1 < NTAP) {
                     load((tap + 1) / TR, (tap + 1) % TR, (tap + 1) % NS, 0);
                 } else {
-                    flip(pbuf ? -PATCH : PATCH);
+                    if constexpr (!ONE) flip(pbuf ? -PATCH : PATCH);
                     load(0, 0, 0, 0);  // (unused after the last unit and before the tail)
                 }
                 mfma(1);
@@ -312,7 +317,7 @@ void conv3_patch_kernel(GemmArgs a) {
             pbuf ^= 1;
         }
         // the dense tail: centre tap, its patch and weights one step ahead
-        for (int st = 0, j = 0; u < uend; ++u, ++j) {
+        for (int st = 0, j = 0; !ONE && u < uend; ++u, ++j) {
             wait_vmcnt_lgkm0<0>();
             __builtin_amdgcn_s_barrier();
             __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -498,13 +503,16 @@ static const PatchCfg kPatch[kNumPatch] = {
     {8, 2, 64, 256, {"conv3_patch_kernel<8,2,64,4,1,9>", "conv3_patch_kernel<8,2,64,4,1,4>"}},
     {8, 2, 64, 256, {"conv3_patch_kernel<8,2,64,4,1,9,9>", ""}},
     {8, 1, 64, 256, {"conv3_patch_kernel<8,1,64,2,2,9,9>", ""}},
-    {8, 1, 32, 128, {"conv3_patch_kernel<8,1,32,2,1,9,9>", ""}}};
+    {8, 1, 32, 128, {"conv3_patch_kernel<8,1,32,2,1,9,9>", ""}},
+    {16, 1, 64, 512, {"conv3_patch_kernel<16,1,64,4,2,9,3,1>", "conv3_patch_kernel<16,1,64,4,2,4,4,1>"}}};
 
 const char* conv_patch_name(int cfg, bool subpix) { return kPatch[cfg].name[subpix]; }
 
 // (four 160-wide weight tiles do not fit the LDS; the shapes with a ring of all nine taps' weights
 // have no four-tap form)
-bool conv_patch_subpix(int cfg) { return cfg != 1 && cfg < 4; }
+bool conv_patch_one_chunk(int cfg) { return cfg == 7; }
+
+bool conv_patch_subpix(int cfg) { return cfg != 1 && (cfg < 4 || cfg == 7); }
 
 int conv_patch_tiles_m(int cfg, const GemmArgs& a) {
     const PatchCfg& p = kPatch[cfg];
@@ -524,6 +532,8 @@ void conv_patch_launch(int cfg, const GemmArgs& a, hipStream_t s) {
         case 6: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 9, 3, 2>), grid, blk, 0, s, a); break;
         case 8: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 9, 9, 1>), grid, blk, 0, s, a); break;
         case 10: SDU_LAUNCH((conv3_patch_kernel<8, 1, 64, 2, 2, 9, 9, 1>), grid, blk, 0, s, a); break;
+        case 15: SDU_LAUNCH((conv3_patch_kernel<16, 1, 64, 4, 2, 4, 4, 4, true>), grid, blk, 0, s, a); break;
+        case 14: SDU_LAUNCH((conv3_patch_kernel<16, 1, 64, 4, 2, 9, 3, 4, true>), grid, blk, 0, s, a); break;
         case 12: SDU_LAUNCH((conv3_patch_kernel<8, 1, 32, 2, 1, 9, 9, 1>), grid, blk, 0, s, a); break;
         case 7: SDU_LAUNCH((conv3_patch_kernel<8, 2, 64, 4, 1, 4, 4, 1>), grid, blk, 0, s, a); break;
     }

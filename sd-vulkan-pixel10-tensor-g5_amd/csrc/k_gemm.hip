@@ -919,7 +919,8 @@ struct Cfg {
 // 4 ..: the patch-resident conv kernel's shapes (k_conv.hip): 16x16 pixels x 128 or 160
 // channels (8 waves, one block per CU), two 8x8 sub-tiles x 80 or 64 channels (4 waves, two);
 // with all nine taps' weights in the ring, for launches of few blocks: two sub-tiles x 64
-// (4 waves, one), one sub-tile x 64 (4 waves, one) or 32 (2 waves, two)
+// (4 waves, one), one sub-tile x 64 (4 waves, one) or 32 (2 waves, two); for convs of 64 input
+// channels, 16x16 pixels x 64 (8 waves, two)
 // Rates and fixed costs of 0..3 from dense GEMMs that give every CU one or two blocks, at
 // K = 512 and 4096 (the difference gives the rate, the rest the fixed cost).  The 64x160
 // tile covers N = 320 with no padded column and M = 8192 with 256 tiles, so it fills the
@@ -934,7 +935,7 @@ struct Cfg {
 // (64x64x512 33 -> 27 us, 2x36x28x640 38 -> 28), the small tiles where a launch is one
 // short round (64x64x64 9.4 -> 7.3 warm, 11.6 -> 7.2 cold); two sub-tiles x 80 with all taps
 // gained 6-10% cold and lost as much warm.
-// 11 ..: gemm_dense_kernel's shapes (k_dense.hip): 256x128 (8 waves, one block per CU),
+// 12 ..: gemm_dense_kernel's shapes (k_dense.hip): 256x128 (8 waves, one block per CU),
 // 128x128, 128x64 (4 waves, two) and 64x64 (4 waves, three), fitted the same way to 2400
 // launches over 50 dense shapes (1 to 65536 rows, K 64 to 6400).
 enum Kind { K_GEMM = 0, K_PATCH = 1, K_DENSE = 2 };
@@ -950,6 +951,7 @@ const Cfg kCfgs[kNumCfg] = {{256, 128, 1, 3.5e12, 3.5e12, 4.5e-6, 1, 1.0, K_GEMM
                             {128, 64, 1, 4.86e12, 4.86e12, 7.1e-6, 1, 1.0, K_PATCH, 4, 0.12e-6},
                             {64, 64, 1, 3.93e12, 3.93e12, 5.4e-6, 1, 1.0, K_PATCH, 5, 0.08e-6},
                             {64, 32, 2, 2.08e12, 3.82e12, 5.0e-6, 1, 1.0, K_PATCH, 6, 0.11e-6},
+                            {256, 64, 2, 7.0e12, 3.8e12, 5.5e-6, 1, 1.0, K_PATCH, 7, 1e-6},
                             {256, 128, 1, 5.5e12, 5.5e12, 4.6e-6, 1, 1.0, K_DENSE, 0, 1.07e-6},
                             {128, 128, 2, 3.76e12, 4.5e12, 3.1e-6, 1, 1.0, K_DENSE, 1, 0.97e-6},
                             {128, 64, 2, 3.57e12, 3.8e12, 2.2e-6, 1, 1.0, K_DENSE, 2, 0.68e-6},
@@ -1019,6 +1021,8 @@ void plan(const GemmArgs& a, int& ci, int& splits, int& kps, bool& fix) {
     for (int c = 0; c < kNumCfg; ++c) {
         const Cfg& g = kCfgs[c];
         if (g.kind != kind || (a.subpix && !conv_patch_subpix(g.shape))) continue;
+        const bool one = patch && conv_patch_one_chunk(g.shape);
+        if (one && (nc != 1 || nkt != ntap)) continue;
         if (kind == K_GEMM) {
             if (a.geglu && g.nt % 128) continue;  // GEGLU pairs 32-column blocks within a 64-wide wave tile
             if (a.stats && !stats_tile_ok(g.mt, a.stats_hw)) continue;
@@ -1027,7 +1031,7 @@ void plan(const GemmArgs& a, int& ci, int& splits, int& kps, bool& fix) {
         const SplitCost& sc = kSplit[kind];
         static const int cand[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
         for (int s : cand) {
-            if (s > 1 && nkt / s < 4) break;
+            if (s > 1 && (nkt / s < 4 || one)) break;
             // (a patch block takes whole chunks of ntap steps, see the kernel's K order)
             int kt_per = ceil_div(nkt, s), se = ceil_div(nkt, kt_per);
             if (patch) {

@@ -167,9 +167,10 @@ hipError_t splitk_reduce_launch(const GemmArgs& a, double bytes, hipStream_t s);
 // The patch-resident 3x3 conv kernel (k_conv.hip): tile shape `cfg` of kNumPatch, for the
 // A_CONV3 GEMMs that gemm_launch sends there (stride 1, no upsample, Cin % 64 == 0, N % 8 ==
 // 0, fp16 or fp32 rows out, any splits).
-constexpr int kNumPatch = 7;
+constexpr int kNumPatch = 8;
 int conv_patch_tiles_m(int cfg, const GemmArgs& a);
-bool conv_patch_subpix(int cfg);  // the shape has a sub-pixel form
+bool conv_patch_subpix(int cfg);     // the shape has a sub-pixel form
+bool conv_patch_one_chunk(int cfg);  // the shape takes convs of one 64-channel chunk only, unsplit
 const char* conv_patch_name(int cfg, bool subpix);
 void conv_patch_launch(int cfg, const GemmArgs& a, hipStream_t s);
 // The dense GEMM kernel with the register epilogue (k_dense.hip): tile shape `cfg` of

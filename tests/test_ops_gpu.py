@@ -370,6 +370,8 @@ def test_conv2d(op_engine, B, H, W, Ci, Co, k, stride, ups, temb, res):
     (1, 33, 39, 64, 72, False, True),      # one sub-tile x 32 columns, one chunk, ragged
     (1, 128, 120, 64, 64, True, True),     # one sub-tile x 64 columns
     (1, 16, 16, 1280, 1280, True, True),   # small tiles, split K
+    (1, 256, 250, 64, 64, True, True),     # one chunk: two 16x16 tiles per CU, a ragged column
+    (3, 203, 190, 64, 72, False, False),   # the same, both directions and the columns ragged
 ])
 def test_conv_patch_tiles(op_engine, B, H, W, Ci, Co, temb, res):
     """Edges of the patch-resident 3x3 kernel's tiles: 8x8 and 16x16 sub-tiles of ragged
