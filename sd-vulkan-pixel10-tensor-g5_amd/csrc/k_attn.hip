@@ -28,7 +28,7 @@
 //   attn_kernel       -- NWAVE query waves share each 64-key K/V tile in LDS
 //                        (long sequences: 64x64 self-attention, 4096 tokens);
 //   attn_wide_kernel  -- the same with 64 queries per wave, scores of the next keys formed
-//                        during the softmax of these (many query blocks, heads of 33..64);
+//                        during the softmax of these (many query blocks, heads of 33..80);
 //   attn_split_kernel -- NSPLIT waves split the keys of one 32-query group and
 //                        merge their partial (max, sum, O) through LDS (short query
 //                        counts, where one wave per 32 queries cannot fill the chip).
@@ -523,9 +523,10 @@ __global__ __launch_bounds__(NWAVE * 64) void attn_kernel(AttnArgs a) {
 // exps of this one's, and their max among its PV products: one straight line of code, the
 // order set by sched_group_barrier, one branch (the reference moves) at its end.
 // d 40, 16 heads x images: 4096 tokens 81 -> 67 us (scale applied in the softmax), 77 -> 62
-// (q pre-scaled); 128 heads x images 513 -> 433 us.
+// (q pre-scaled); 128 heads x images 513 -> 433 us.  d 80 (one wave per SIMD, 416
+// registers), 1024 tokens, 128 heads x images 79 -> 66 us.
 template <int KS, int MTD, bool LSUM, bool OFS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn_wide_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KS <= 4 ? 2 : 1))) void attn_wide_kernel(AttnArgs a) {
     constexpr int KT = 64, G = 2;
     constexpr int VSTR = ((MTD * 32 - 16 + 63) / 64) * 64 + 16;  // as attn_kernel's TRV
     constexpr int KSTR = KS * 16 + 8, KTILE = KT * KSTR, VTILE = KT * VSTR, NTH = 256;
@@ -729,7 +730,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 if (i < KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
-                if (i < 4) __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+                if (i < (32 - 24 / (KS * G) * KS * G) / 2) __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
             }
         }
         if (__ballot(up)) rebase(nxt, mx, false);
@@ -1027,22 +1028,24 @@ static AttnPlan attn_plan(const AttnArgs& a) {
     // with two, 0.158 with four).  Fewer query waves (e.g. 1024 queries x 16 heads), and
     // short key sequences (cross-attention over the 77 context tokens), go to the
     // key-split kernel: its extra waves, or not staging a few K/V tiles per block, win.
+    // 64 queries per wave for heads of 33..80 where their 256-query blocks cover enough of the CUs.
+    // Time against the narrow tiles', d 40 / d 64: 128 blocks 0.9-1.1 / 0.8-1.0, 144 to 256
+    // 0.78-0.87 / 0.81-0.98, 257 to 320 (a short second round) 1.02-1.08 / 0.78-1.05, above
+    // 0.45-0.97 / 0.7-0.9; d 80 from 96 blocks on 0.43-0.98.  Heads up to 32 have half the PV work
+    // per exp and lose (0.9-1.4); up to 128 keys the loop is too short (d 80 0.7-1.2).
+    const int64_t nwide = ((a.Sq + 255) / 256) * bh;
+    if (a.Sk > 128 && !a.causal &&
+        (KS == 5 ? nwide >= 96 && qwaves >= 768
+                 : (KS == 3 || KS == 4) && nwide >= 144 && (nwide <= 256 || nwide > 320) && qwaves >= 1024)) {
+        p.shared = p.wide = true;
+        p.ofs = a.q_log2 && a.d < KS * 16;
+        p.grid = dim3((a.Sq + 255) / 256, a.heads, a.B);
+        return p;
+    }
     if (qwaves >= 1024 && a.Sk > 128 && !a.causal) {
         p.shared = true;
         p.nw = (a.d > 48 && a.d <= 128 && ((a.Sq + 127) / 128) * bh < 512) ? 8 : 4;
         p.grid = dim3((a.Sq + p.nw * 32 - 1) / (p.nw * 32), a.heads, a.B);
-        // 64 queries per wave for heads of 33..64 where their 256-query blocks cover more than
-        // half of the CUs (144 blocks and up) and leave no short second round (257..320 of 256
-        // CUs).  Time against the narrow tiles', d 40 / d 64: 128 blocks 0.9-1.1 / 0.8-1.0,
-        // 144 to 256 0.78-0.87 / 0.81-0.98, 257 to 320 1.02-1.08 / 0.78-1.05, above 0.45-0.97 /
-        // 0.7-0.9.  Heads up to 32 have half the PV work per exp and lose (0.9-1.4).
-        const long nwide = (long)((a.Sq + 255) / 256) * bh;
-        if ((KS == 3 || KS == 4) && nwide >= 144 && (nwide <= 256 || nwide > 320)) {
-            p.wide = true;
-            p.ofs = a.q_log2 && a.d < KS * 16;
-            p.grid = dim3((a.Sq + 255) / 256, a.heads, a.B);
-            return p;
-        }
         // 128-key tiles for heads <= 48 when every block is resident at once (two per CU):
         // d40 at 4096 tokens, B=2, 0.44 ms per forward against 0.46 with 64-key tiles;
         // on larger grids they lose (0.24 ms more at 9216 tokens, 0.31 ms at B=16)
@@ -1091,7 +1094,7 @@ static void launch_cfg(const AttnArgs& a0, hipStream_t s) {
     const double flops = 4.0 * bh * a.Sq * a.Sk * a.d;
     const double bytes = 2.0 * bh * a.d * (2.0 * a.Sq + 2.0 * a.Sk);
     char name[48];
-    if constexpr (KS == 3 || KS == 4) {
+    if constexpr (KS >= 3 && KS <= 5) {
         if (p.wide) {
             snprintf(name, sizeof name, "attn_wide_kernel<%d,%d,%d,%d>", KS, MTD, (int)LSUM, (int)p.ofs);
             launch_timed(name, flops, bytes, [&] {
