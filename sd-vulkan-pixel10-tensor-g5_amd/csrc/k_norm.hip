@@ -5,7 +5,8 @@
 // The reference reduces one group per 256-thread workgroup; here the image is
 // split into pixel chunks so the whole chip streams the tensor:
 //   pass 1 (stats): each block reads a stretch of pixels x all channels with 16-byte
-//     loads, reduces per-group sum and sum of squares in fp32 and stores them.
+//     loads, reduces per-group sum and sum of squares (of the values less the group's first
+//     one) in fp32 and stores them.
 //   pass 2 (apply): adds the partials up; mean = S1/N, var = S2/N - mean^2 in fp64; then
 //     y = x * a_c + b_c (a_c = rstd_g gamma_c, b_c = beta_c - mean_g a_c),
 //     optional SiLU, 16-byte loads and stores.
@@ -61,9 +62,16 @@ __device__ __forceinline__ GnSrc gn_src(const f16* x, const f16* x2, int C1, int
     return ch < C1 ? GnSrc{x + ch, C1} : GnSrc{x2 + (ch - C1), C2};
 }
 
-// Per-group (sum, sum of squares) of a block's pixels, stored as part[b][block][g]: no atomics
+// The value a group's statistics are shifted by, so that its one-pass variance does not cancel when
+// the mean dwarfs the spread: its first channel at the image's first pixel.
+__device__ __forceinline__ float gn_shift(const f16* x, const f16* x2, int C1, int C2, int64_t pix0, int c0) {
+    const GnSrc s = gn_src(x, x2, C1, C2, c0);
+    return (float)s.p[pix0 * s.ld];
+}
+
+// Per-group (sum, sum of squares) of a block's pixels less the group's shift, stored as part[b][block][g]: no atomics
 // and nothing to clear.  (With fp64 atomics per group from blocks of 8192 elements and the clear
-// before them, 2 x 4096 x 960 took 25 + 3.6 us; it takes 5.2.)  8 pixels per thread and round, all in flight,
+// before them, 2 x 4096 x 960 took 25 + 3.6 us; it takes 5.6.)  8 pixels per thread and round, all in flight,
 // added as a tree.
 __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, const f16* x2, int C1, int C2, int HW,
                                                               int P, int G, float2* part) {
@@ -76,22 +84,25 @@ __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, cons
     if (ph < R) {
         const GnSrc src = gn_src(x, x2, C1, C2, o * 8);
         const f16* base = src.p + (int64_t)b * HW * src.ld;
-        float a[8], q[8];
+        float a[8], q[8], sh[8];
+        int c0 = o * 8 / cpg * cpg;  // first channel of channel o * 8's group
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { a[e] = 0.f; q[e] = 0.f; }
+        for (int e = 0; e < 8; ++e) {
+            a[e] = 0.f;
+            q[e] = 0.f;
+            if (o * 8 + e >= c0 + cpg) c0 += cpg;
+            sh[e] = gn_shift(x, x2, C1, C2, (int64_t)b * HW, c0);
+        }
         for (int p = p0 + ph; p < pe; p += U * R) {
             uint4 raw[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) raw[u] = *(const uint4*)(base + (int64_t)min(p + u * R, pe - 1) * src.ld);
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (p + u * R >= pe) raw[u] = make_uint4(0, 0, 0, 0);
-#pragma unroll
             for (int e = 0; e < 8; ++e) {
                 float f[U], g[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    f[u] = (float)((const f16*)&raw[u])[e];
+                    f[u] = p + u * R < pe ? (float)((const f16*)&raw[u])[e] - sh[e] : 0.f;
                     g[u] = f[u] * f[u];
                 }
 #pragma unroll
@@ -133,7 +144,7 @@ __device__ __forceinline__ float silu_f(float x) { return x * __builtin_amdgcn_r
 // Apply y = act((x - mean_g) * rstd_g * gamma + beta): block (i, b) does the pixels of GnGeom's
 // block i of image b, GNA_U pixels per thread and round, the next round's loads in flight
 // during this one's arithmetic and the first round's during the statistics.
-// CST = false: the groups' sums from gn_stats_kernel's partials, part[b][npart][G].
+// CST = false: the groups' sums from gn_stats_kernel's partials, part[b][npart][G] (shifted).
 // CST = true: from per-channel sums st1 [B][C1][2] and st2 [B][C2][2] kept by the GEMM epilogues
 // that produced x and x2.
 static constexpr int GNA_U = 4;
@@ -160,6 +171,7 @@ __global__ __launch_bounds__(GN_THREADS) void gn_apply_kernel(const f16* x, cons
     __shared__ double2 red[CST ? 1 : GN_THREADS];
     // 16 threads add up each group
     const int g = tid / 16, sub = tid % 16;
+    const float shift = CST ? 0.f : gn_shift(x, x2, C1, C2, (int64_t)b * HW, min(g, G - 1) * cpg);
     double ga = 0.0, gq = 0.0;
     if constexpr (CST) {
         if (g < G) {
@@ -215,7 +227,7 @@ __global__ __launch_bounds__(GN_THREADS) void gn_apply_kernel(const f16* x, cons
         const double n = (double)HW * cpg;
         const double mean = ga / n;
         const double var = fmax(gq / n - mean * mean, 0.0);
-        s_mean[g] = (float)mean;
+        s_mean[g] = (float)(mean + (CST ? 0.f : shift));
         s_rstd[g] = (float)(1.0 / sqrt(var + (double)eps));
     }
     __syncthreads();

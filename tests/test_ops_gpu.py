@@ -76,6 +76,13 @@ def test_groupnorm_two_pass(op_engine, B, H, W, C1, C2, silu):
     test_groupnorm(op_engine, B, H, W, C1, C2, silu)
 
 
+def test_groupnorm_two_pass_large_mean(op_engine):
+    """test_groupnorm_large_mean's bound for the statistics and apply passes (slabs of 92160 elements;
+    3 channels per group)."""
+    test_groupnorm_large_mean(op_engine, 2, 96, 96, 320, False)
+    test_groupnorm_large_mean(op_engine, 16, 24, 24, 96, True)
+
+
 @pytest.mark.parametrize("B,H,W,C,silu", [(2, 32, 32, 640, True), (2, 16, 16, 1280, False)])
 def test_groupnorm_large_mean(op_engine, B, H, W, C, silu):
     """Groups whose mean is 100x their spread (the single-kernel path sums x minus the
