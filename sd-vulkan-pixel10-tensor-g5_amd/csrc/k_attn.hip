@@ -1032,9 +1032,11 @@ static AttnPlan attn_plan(const AttnArgs& a) {
     // Time against the narrow tiles', d 40 / d 64: 128 blocks 0.9-1.1 / 0.8-1.0, 144 to 256
     // 0.78-0.87 / 0.81-0.98, 257 to 320 (a short second round) 1.02-1.08 / 0.78-1.05, above
     // 0.45-0.97 / 0.7-0.9; d 80 from 96 blocks on 0.43-0.98.  Heads up to 32 have half the PV work
-    // per exp and lose (0.9-1.4); up to 128 keys the loop is too short (d 80 0.7-1.2).
+    // per exp and lose (0.9-1.4).  With 65 to 128 keys (against the key-split kernel) the loop is two
+    // tiles: d 40 and 64 gain from 1024 blocks on (0.76-0.94; 576 blocks, 2.25 rounds, 0.93-1.2), d 80
+    // does not (0.9-1.2).
     const int64_t nwide = ((a.Sq + 255) / 256) * bh;
-    if (a.Sk > 128 && !a.causal &&
+    if (a.Sk > (KS <= 4 && nwide >= 1024 ? 64 : 128) && !a.causal &&
         (KS == 5 ? nwide >= 96 && qwaves >= 768
                  : (KS == 3 || KS == 4) && nwide >= 144 && (nwide <= 256 || nwide > 320) && qwaves >= 1024)) {
         p.shared = p.wide = true;

@@ -613,6 +613,8 @@ def test_attention_q_log2_reference_moves(op_engine, B):
     (41, 8, 290, 256, 40),   # whole tiles; two rounds of blocks
     (12, 8, 230, 129, 80),   # 96 query blocks, the fewest of this head size; one wave per SIMD
     (10, 8, 300, 350, 72),   # a spare dimension in the fifth k-step
+    (64, 16, 130, 65, 40),   # two key tiles, the second of one key
+    (64, 16, 256, 77, 64),   # cross-attention keys, row sums outside the MFMA
 ])
 def test_attention_wide(op_engine, B, heads, Sq, Sk, d):
     """Edges of the 64-queries-per-wave kernel's query blocks and key steps, with either form of the scale."""
