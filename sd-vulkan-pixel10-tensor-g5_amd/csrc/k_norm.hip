@@ -6,7 +6,7 @@
 // split into pixel chunks so the whole chip streams the tensor:
 //   pass 1 (stats): each block reads a stretch of pixels x all channels with 16-byte
 //     loads, reduces per-group sum and sum of squares (of the values less the group's first
-//     one) in fp32 and stores them.
+//     one) in fp32 and stores them as mean and squared deviations.
 //   pass 2 (apply): adds the partials up; mean = S1/N, var = S2/N - mean^2 in fp64; then
 //     y = x * a_c + b_c (a_c = rstd_g gamma_c, b_c = beta_c - mean_g a_c),
 //     optional SiLU, 16-byte loads and stores.
@@ -69,10 +69,10 @@ __device__ __forceinline__ float gn_shift(const f16* x, const f16* x2, int C1, i
     return (float)s.p[pix0 * s.ld];
 }
 
-// Per-group (sum, sum of squares) of a block's pixels less the group's shift, stored as part[b][block][g]: no atomics
-// and nothing to clear.  (With fp64 atomics per group from blocks of 8192 elements and the clear
-// before them, 2 x 4096 x 960 took 25 + 3.6 us; it takes 5.6.)  8 pixels per thread and round, all in flight,
-// added as a tree.
+// Per-group (mean, sum of squared deviations from it) of a block's pixels, summed less the group's
+// shift and stored as part[b][block][g]: no atomics and nothing to clear.  (With fp64 atomics per
+// group from blocks of 8192 elements and the clear before them, 2 x 4096 x 960 took 25 + 3.6 us;
+// it takes 5.6.)  8 pixels per thread and round, all in flight, added as a tree.
 __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, const f16* x2, int C1, int C2, int HW,
                                                               int P, int G, float2* part) {
     constexpr int U = 8;
@@ -135,7 +135,11 @@ __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, cons
         ga += __shfl_xor(ga, off);
         gq += __shfl_xor(gq, off);
     }
-    if (tid % 16 == 0) part[((int64_t)b * gridDim.x + blockIdx.x) * G + g] = make_float2(ga, gq);
+    if (tid % 16 == 0) {
+        const double m = (double)ga / ((double)(pe - p0) * cpg);
+        part[((int64_t)b * gridDim.x + blockIdx.x) * G + g] =
+            make_float2((float)(m + gn_shift(x, x2, C1, C2, (int64_t)b * HW, g * cpg)), (float)(gq - ga * m));
+    }
 }
 
 // (v_rcp_f32 is within 1 ulp: an error of 2^-24 in front of the fp16 rounding)
@@ -144,7 +148,9 @@ __device__ __forceinline__ float silu_f(float x) { return x * __builtin_amdgcn_r
 // Apply y = act((x - mean_g) * rstd_g * gamma + beta): block (i, b) does the pixels of GnGeom's
 // block i of image b, GNA_U pixels per thread and round, the next round's loads in flight
 // during this one's arithmetic and the first round's during the statistics.
-// CST = false: the groups' sums from gn_stats_kernel's partials, part[b][npart][G] (shifted).
+// CST = false: the groups' statistics from gn_stats_kernel's partials, part[b][npart][G] of npart
+// blocks of SP pixels (the last one the rest), put together as sums in fp64.  (y may be x: a block
+// reads no pixels but its own.)
 // CST = true: from per-channel sums st1 [B][C1][2] and st2 [B][C2][2] kept by the GEMM epilogues
 // that produced x and x2.
 static constexpr int GNA_U = 4;
@@ -153,7 +159,7 @@ template <bool CST>
 __global__ __launch_bounds__(GN_THREADS) void gn_apply_kernel(const f16* x, const f16* x2, int C1, int C2,
                                                               const f16* gamma, const f16* beta, f16* y, int HW,
                                                               int P, int G, float eps, int silu, const float2* part,
-                                                              int npart, const double* st1, const double* st2) {
+                                                              int npart, int SP, const double* st1, const double* st2) {
     const int C = C1 + C2, V = C / 8, cpg = C / G, R = GN_THREADS / V;
     const int b = blockIdx.y, tid = threadIdx.x;
     const int ph = tid / V, o = tid - ph * V;
@@ -171,7 +177,6 @@ __global__ __launch_bounds__(GN_THREADS) void gn_apply_kernel(const f16* x, cons
     __shared__ double2 red[CST ? 1 : GN_THREADS];
     // 16 threads add up each group
     const int g = tid / 16, sub = tid % 16;
-    const float shift = CST ? 0.f : gn_shift(x, x2, C1, C2, (int64_t)b * HW, min(g, G - 1) * cpg);
     double ga = 0.0, gq = 0.0;
     if constexpr (CST) {
         if (g < G) {
@@ -202,9 +207,10 @@ __global__ __launch_bounds__(GN_THREADS) void gn_apply_kernel(const f16* x, cons
                 for (int u = 0; u < 4; ++u) v[u] = pp[(int64_t)min(i0 + u * NP, npart - 1) * G];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    const bool use = i0 + u * NP < npart;
-                    ga += use ? (double)v[u].x : 0.0;
-                    gq += use ? (double)v[u].y : 0.0;
+                    const int i = i0 + u * NP;
+                    const double s = (double)(min(SP, HW - i * SP) * cpg) * (double)v[u].x;
+                    ga += i < npart ? s : 0.0;
+                    gq += i < npart ? fma(s, (double)v[u].x, (double)v[u].y) : 0.0;
                 }
             }
         }
@@ -227,7 +233,7 @@ __global__ __launch_bounds__(GN_THREADS) void gn_apply_kernel(const f16* x, cons
         const double n = (double)HW * cpg;
         const double mean = ga / n;
         const double var = fmax(gq / n - mean * mean, 0.0);
-        s_mean[g] = (float)(mean + (CST ? 0.f : shift));
+        s_mean[g] = (float)mean;
         s_rstd[g] = (float)(1.0 / sqrt(var + (double)eps));
     }
     __syncthreads();
@@ -467,7 +473,7 @@ hipError_t groupnorm_launch(const f16* x, const f16* x2, int C1, int C2, const f
     if (e != hipSuccess) return e;
     launch_timed("gn_apply_kernel<0>", 0.0, 2.0 * xbytes, [&] {
         SDU_LAUNCH(gn_apply_kernel<false>, dim3(ga.nblk, B), dim3(GN_THREADS), 0, s, x, x2, C1, C2, gamma, beta, y,
-                   HW, ga.P, G, eps, silu, (const float2*)part, gs.nblk, (const double*)nullptr, (const double*)nullptr);
+                   HW, ga.P, G, eps, silu, (const float2*)part, gs.nblk, gs.P, (const double*)nullptr, (const double*)nullptr);
     });
     return hipGetLastError();
 }
@@ -483,7 +489,7 @@ hipError_t groupnorm_apply_stats_launch(const f16* x, const f16* x2, int C1, int
     const GnGeom ga = gn_geom(B, HW, C, GNA_BLOCKS);
     launch_timed("gn_apply_kernel<1>", 0.0, 2.0 * xbytes, [&] {
         SDU_LAUNCH(gn_apply_kernel<true>, dim3(ga.nblk, B), dim3(GN_THREADS), 0, s, x, x2, C1, C2, gamma, beta, y, HW,
-                   ga.P, G, eps, silu, (const float2*)nullptr, 0, st1, st2);
+                   ga.P, G, eps, silu, (const float2*)nullptr, 0, 0, st1, st2);
     });
     return hipGetLastError();
 }

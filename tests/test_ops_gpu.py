@@ -83,6 +83,23 @@ def test_groupnorm_two_pass_large_mean(op_engine):
     test_groupnorm_large_mean(op_engine, 16, 24, 24, 96, True)
 
 
+@pytest.mark.parametrize("B,H,W,C", [(2, 96, 96, 320), (3, 24, 25, 96), (1, 97, 31, 2560)])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_groupnorm_two_pass_in_place(op_engine, B, H, W, C, noalloc):
+    """y = x: the apply blocks read nothing of x that another block writes, so the result is that of a
+    separate output, bit for bit."""
+    say(f"groupnorm in place B={B} {H}x{W} C={C} noalloc={noalloc}")
+    import sdu
+    e = op_engine
+    gn = getattr(sdu.load(), "sdu_groupnorm_noalloc" if noalloc else "sdu_groupnorm")
+    x = r16((B, H * W, C), 12, 2.0, 5.0).astype(np.float16)
+    tg, tb = e.upload(r16((C,), 2, 0.3, 1.0).astype(np.float16)), e.upload(r16((C,), 3, 0.3).astype(np.float16))
+    tx, ty = e.upload(x), e.tensor((B, H * W, C))
+    for out in (ty, tx):
+        e._check(gn(e.h, tx.h, None, tg.h, tb.h, out.h, B, H * W, C, 0, 32, 1e-5, 1))
+    np.testing.assert_array_equal(tx.numpy(), ty.numpy())
+
+
 @pytest.mark.parametrize("B,H,W,C,silu", [(2, 32, 32, 640, True), (2, 16, 16, 1280, False)])
 def test_groupnorm_large_mean(op_engine, B, H, W, C, silu):
     """Groups whose mean is 100x their spread (the single-kernel path sums x minus the
