@@ -5,8 +5,8 @@
 // The reference reduces one group per 256-thread workgroup; here the image is
 // split into pixel chunks so the whole chip streams the tensor:
 //   pass 1 (stats): each block reads a stretch of pixels x all channels with 16-byte
-//     loads, reduces per-group sum and sum of squares (of the values less the group's first
-//     one) in fp32 and stores them as mean and squared deviations.
+//     loads, reduces per-group sum and sum of squares in fp64 and stores them as mean and
+//     squared deviations.
 //   pass 2 (apply): adds the partials up; mean = S1/N, var = S2/N - mean^2 in fp64; then
 //     y = x * a_c + b_c (a_c = rstd_g gamma_c, b_c = beta_c - mean_g a_c),
 //     optional SiLU, 16-byte loads and stores.
@@ -62,17 +62,13 @@ __device__ __forceinline__ GnSrc gn_src(const f16* x, const f16* x2, int C1, int
     return ch < C1 ? GnSrc{x + ch, C1} : GnSrc{x2 + (ch - C1), C2};
 }
 
-// The value a group's statistics are shifted by, so that its one-pass variance does not cancel when
-// the mean dwarfs the spread: its first channel at the image's first pixel.
-__device__ __forceinline__ float gn_shift(const f16* x, const f16* x2, int C1, int C2, int64_t pix0, int c0) {
-    const GnSrc s = gn_src(x, x2, C1, C2, c0);
-    return (float)s.p[pix0 * s.ld];
-}
-
-// Per-group (mean, sum of squared deviations from it) of a block's pixels, summed less the group's
-// shift and stored as part[b][block][g]: no atomics and nothing to clear.  (With fp64 atomics per
-// group from blocks of 8192 elements and the clear before them, 2 x 4096 x 960 took 25 + 3.6 us;
-// it takes 5.6.)  8 pixels per thread and round, all in flight, added as a tree.
+// Per-group (mean, sum of squared deviations from it) of a block's pixels, stored as
+// part[b][block][g]: no atomics and nothing to clear.  The sums are fp64: fp32 ones lose the variance
+// of groups whose mean dwarfs their spread, and fp32 ones less a value of the group that of groups
+// where that value is an outlier (relative error 1e-3 at 300 spreads); the conversions are no more
+// instructions than the shift was.  8 pixels per thread and round, all in flight.  Bound by latency
+// at the networks' sizes: 2 x 4096 x 960 with its apply 16.8 us (17.3 to 17.6 with shifted fp32 sums,
+// whose shift was one more dependent load; 37.1 with fp64 atomics per 8192 elements and their clear).
 __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, const f16* x2, int C1, int C2, int HW,
                                                               int P, int G, float2* part) {
     constexpr int U = 8;
@@ -80,51 +76,42 @@ __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, cons
     const int b = blockIdx.y, tid = threadIdx.x;
     const int ph = tid / V, o = tid - ph * V;
     const int p0 = blockIdx.x * P, pe = min(HW, p0 + P);
-    __shared__ float s1[GN_THREADS * 8], s2[GN_THREADS * 8];  // [R][C]
+    __shared__ __attribute__((aligned(16))) double s1[GN_THREADS * 8], s2[GN_THREADS * 8];  // [R][C]
     if (ph < R) {
         const GnSrc src = gn_src(x, x2, C1, C2, o * 8);
         const f16* base = src.p + (int64_t)b * HW * src.ld;
-        float a[8], q[8], sh[8];
-        int c0 = o * 8 / cpg * cpg;  // first channel of channel o * 8's group
+        double a[8], q[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            a[e] = 0.f;
-            q[e] = 0.f;
-            if (o * 8 + e >= c0 + cpg) c0 += cpg;
-            sh[e] = gn_shift(x, x2, C1, C2, (int64_t)b * HW, c0);
-        }
+        for (int e = 0; e < 8; ++e) { a[e] = 0.0; q[e] = 0.0; }
         for (int p = p0 + ph; p < pe; p += U * R) {
             uint4 raw[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) raw[u] = *(const uint4*)(base + (int64_t)min(p + u * R, pe - 1) * src.ld);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float f[U], g[U];
+            for (int u = 0; u < U; ++u)
+                if (p + u * R >= pe) raw[u] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    f[u] = p + u * R < pe ? (float)((const f16*)&raw[u])[e] - sh[e] : 0.f;
-                    g[u] = f[u] * f[u];
+                    const double f = (float)((const f16*)&raw[u])[e];
+                    a[e] += f;
+                    q[e] = fma(f, f, q[e]);
                 }
-#pragma unroll
-                for (int n = U / 2; n > 0; n >>= 1)
-#pragma unroll
-                    for (int u = 0; u < n; ++u) { f[u] += f[u + n]; g[u] += g[u + n]; }
-                a[e] += f[0];
-                q[e] += g[0];
-            }
         }
-        float* w1 = s1 + ph * C + o * 8;
-        float* w2 = s2 + ph * C + o * 8;
-        *(float4*)w1 = make_float4(a[0], a[1], a[2], a[3]);
-        *(float4*)(w1 + 4) = make_float4(a[4], a[5], a[6], a[7]);
-        *(float4*)w2 = make_float4(q[0], q[1], q[2], q[3]);
-        *(float4*)(w2 + 4) = make_float4(q[4], q[5], q[6], q[7]);
+        double2* w1 = (double2*)(s1 + ph * C + o * 8);
+        double2* w2 = (double2*)(s2 + ph * C + o * 8);
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            w1[e / 2] = make_double2(a[e], a[e + 1]);
+            w2[e / 2] = make_double2(q[e], q[e + 1]);
+        }
     }
     __syncthreads();
     // 16 threads per group
     const int g = tid / 16;
     if (g >= G) return;
-    float ga = 0.f, gq = 0.f;
+    double ga = 0.0, gq = 0.0;
     for (int r = 0; r < R; ++r)
         for (int i = tid % 16; i < cpg; i += 16) {
             ga += s1[r * C + g * cpg + i];
@@ -135,11 +122,8 @@ __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, cons
         ga += __shfl_xor(ga, off);
         gq += __shfl_xor(gq, off);
     }
-    if (tid % 16 == 0) {
-        const double m = (double)ga / ((double)(pe - p0) * cpg);
-        part[((int64_t)b * gridDim.x + blockIdx.x) * G + g] =
-            make_float2((float)(m + gn_shift(x, x2, C1, C2, (int64_t)b * HW, g * cpg)), (float)(gq - ga * m));
-    }
+    const double mean = ga / ((double)(pe - p0) * cpg);
+    if (tid % 16 == 0) part[((int64_t)b * gridDim.x + blockIdx.x) * G + g] = make_float2((float)mean, (float)(gq - ga * mean));
 }
 
 // (v_rcp_f32 is within 1 ulp: an error of 2^-24 in front of the fp16 rounding)

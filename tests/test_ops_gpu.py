@@ -100,6 +100,33 @@ def test_groupnorm_two_pass_in_place(op_engine, B, H, W, C, noalloc):
     np.testing.assert_array_equal(tx.numpy(), ty.numpy())
 
 
+@pytest.mark.parametrize("B,H,W,C", [(2, 96, 96, 320), (1, 64, 64, 960), (8, 96, 96, 96)])
+@pytest.mark.parametrize("v", [300.0, 10000.0, -10000.0])
+def test_groupnorm_two_pass_outlier(op_engine, B, H, W, C, v):
+    """N(0, 1) groups whose first value is v, on the statistics and apply passes: the least-squares
+    scale of each group's output against a 64-bit GroupNorm's, without the outlier, is 1 - (relative
+    error of the variance) / 2.  Bound 1.5e-5: an fp16 output's rounding is 2.0e-4 rms of its value,
+    which over the 27648 values of the smallest group leaves 2.1e-6 at one deviation, 7e-6 in the worst
+    of 256 groups; an fp32 rounding adds 1e-7.  A pass that shifts fp32 sums by the outlier is off by
+    2.5e-4 and up."""
+    say(f"groupnorm outlier B={B} {H}x{W} C={C} v={v}")
+    e = op_engine
+    HW, G = H * W, 32
+    x = r16((B, HW, C), 13).reshape(B, HW, G, C // G)
+    x[:, 0, :, 0] = v
+    one, zero = e.upload(np.ones(C, np.float16)), e.upload(np.zeros(C, np.float16))
+    ty = e.tensor((B, HW, C))
+    e.groupnorm(e.upload(x.reshape(B, HW, C).astype(np.float16)), one, zero, ty, B, HW, C, 0, silu=False)
+    got = ty.numpy().astype(np.float64).reshape(x.shape)
+    xd = x.astype(np.float64)
+    ref = (xd - xd.mean((1, 3), keepdims=True)) / np.sqrt(xd.var((1, 3), keepdims=True) + 1e-5)
+    got[:, 0, :, 0] = ref[:, 0, :, 0] = 0.0
+    got, ref = (a - a.mean((1, 3), keepdims=True) for a in (got, ref))
+    scale = (got * ref).sum((1, 3)) / (ref * ref).sum((1, 3))
+    say(f"  largest scale error {np.abs(scale - 1).max():.1e}")
+    assert np.abs(scale - 1).max() < 1.5e-5
+
+
 @pytest.mark.parametrize("B,H,W,C,silu", [(2, 32, 32, 640, True), (2, 16, 16, 1280, False)])
 def test_groupnorm_large_mean(op_engine, B, H, W, C, silu):
     """Groups whose mean is 100x their spread (the single-kernel path sums x minus the
