@@ -503,9 +503,12 @@ static int dense_ep(const GemmArgs& a) {
 }
 
 // Whole K tiles, 8-column chunks, 16-row fragments that lie in one image (channel statistics),
-// and the combinations of epilogue options that have a variant.
+// and the combinations of epilogue options that have a variant.  A tile's 256 output (and
+// residual) rows must lie within 1 GiB: the epilogue's byte offsets are 32 bits, and a column past N
+// gets one of 1 GiB and up to be past the rows.  (gemm_kernel's are 64 bits.)
 bool dense_ok(const GemmArgs& a) {
     if (a.amode != A_DENSE || a.K % 64 || (a.A2 && a.K1 % 64) || a.N % 8) return false;
+    if (256LL * a.ldc * (a.out_mode == OUT_F32 ? 4 : 2) > 1 << 30 || (a.res && 256LL * a.ldr * 2 > 1 << 30)) return false;
     if (a.geglu) return !a.res && !a.act && a.out_mode == OUT_F16;
     if (a.ln_part || a.row_part || a.stats)
         return (!a.act || (a.ln_part && a.act == ACT_QUICK_GELU)) && a.out_mode == OUT_F16 && !(a.row_part && a.stats) &&

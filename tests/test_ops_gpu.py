@@ -309,6 +309,42 @@ def test_matmul_dense_tiles(op_engine, M, N, K, K2, bias, res, geglu, f32):
     test_matmul(op_engine, M, N, K, K2, bias, res, geglu, f32)
 
 
+def kernels_of(e, f):
+    """The kernels that f's op-level calls launch, by name."""
+    e.profile_ops(True)
+    try:
+        f()
+    finally:
+        prof, _ = e.profile_ops(False)
+    return {n[2:] for n in prof if n.startswith("k:")}
+
+
+@pytest.mark.parametrize("N,f32,kernel", [
+    (2097144, False, "gemm_dense_kernel"),  # 256 rows of almost 1 GiB, a last tile of 120 columns
+    (2097160, False, "gemm_kernel"),
+    (524296, True, "gemm_dense_kernel"),    # a last tile of 8 columns
+    (1048584, True, "gemm_kernel"),
+])
+def test_matmul_wide_rows(op_engine, N, f32, kernel):
+    """Rows so wide that a tile's output spans the dense kernel's 32-bit offsets: its column chunks
+    past N must not land in another row, and wider rows take the kernel with 64-bit offsets."""
+    import sdu
+    say(f"matmul wide rows N={N} f32={f32}")
+    e = op_engine
+    M, K, n0 = 256, 64, 4099
+    a, w = r16((M, K), 55), r16((n0, K), 56, 0.1)
+    ty = e.tensor((M, N), sdu.SDU_F32 if f32 else 1)
+    tw = e.upload(np.tile(w.astype(np.float16), (N // n0 + 1, 1))[:N])
+    ta = e.upload(a.astype(np.float16))
+    names = kernels_of(e, lambda: e.matmul(ta, tw, ty, M, N, K, flags=sdu.SDU_EPI_OUT_F32 if f32 else 0))
+    assert [n.split("<")[0] for n in names] == [kernel], names
+    ref, got = a @ w.T, ty.numpy()
+    tol = 1e-5 if f32 else 2.0**-11 * np.abs(ref).max() + 1e-5  # fp32 sums of 64 terms, the fp16 rounding
+    for c in range(0, N, n0):
+        g = got[:, c:c + n0].astype(np.float32)
+        assert np.abs(g - ref[:, :g.shape[1]]).max() <= tol, c
+
+
 def test_geglu_gate_range(op_engine):
     """The gate's GELU over fp16's range: exact zero below about -6, the identity above, infinity
     kept.  A&S 7.1.26's 1.5e-7 on erf bounds the absolute error by 7.5e-8 |b|; the rest is the
