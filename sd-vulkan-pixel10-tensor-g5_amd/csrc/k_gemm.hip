@@ -1002,8 +1002,9 @@ bool patch_ok(const GemmArgs& a) {
            a.out_mode != OUT_F32_NCHW && !a.geglu && !a.row_part && !a.ln_part;
 }
 
-// The epilogue keeps output statistics for two images per tile: the MT rows of a tile
-// (MT-aligned) must not reach a third image.
+// The epilogues of gemm_kernel and gemm_dense_kernel keep output statistics for two images per
+// tile: the MT rows of a tile (MT-aligned) must not reach a third image.  (A patch tile's
+// sub-tiles are of one image each.)
 bool stats_tile_ok(int mt, int hw) { return hw >= mt || mt == 2 * hw; }
 
 // Pick the tile shape and split-K factor with the lowest modelled time.  Blocks are
@@ -1023,10 +1024,8 @@ void plan(const GemmArgs& a, int& ci, int& splits, int& kps, bool& fix) {
         if (g.kind != kind || (a.subpix && !conv_patch_subpix(g.shape))) continue;
         const bool one = patch && conv_patch_one_chunk(g.shape);
         if (one && (nc != 1 || nkt != ntap)) continue;
-        if (kind == K_GEMM) {
-            if (a.geglu && g.nt % 128) continue;  // GEGLU pairs 32-column blocks within a 64-wide wave tile
-            if (a.stats && !stats_tile_ok(g.mt, a.stats_hw)) continue;
-        }
+        if (kind == K_GEMM && a.geglu && g.nt % 128) continue;  // GEGLU pairs 32-column blocks within a 64-wide wave tile
+        if (!patch && a.stats && !stats_tile_ok(g.mt, a.stats_hw)) continue;
         const int tiles = cfg_tiles(c, a);
         const SplitCost& sc = kSplit[kind];
         static const int cand[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
@@ -1161,7 +1160,7 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
                                (a.A2 && 2 * (int64_t)a.M * a.lda2 > lim) || (a.A3 && 2 * (int64_t)a.M * a.lda3 > lim)))
         return hipErrorInvalidValue;
     if (a.stats && (a.out_mode != OUT_F16 || a.geglu || (a.N & 7) || a.stats_hw < 64 ||
-                    (g.kind == K_GEMM ? !stats_tile_ok(g.mt, a.stats_hw) : g.kind == K_PATCH && a.stats_hw != a.Ho * a.Wo)))
+                    (g.kind == K_PATCH ? a.stats_hw != a.Ho * a.Wo : !stats_tile_ok(g.mt, a.stats_hw))))
         return hipErrorInvalidValue;
     const dim3 grid(cfg_tiles(ci, a), 1, splits);
     // algorithmic traffic: A once (the conv source image, not its im2col), W once, output
