@@ -91,10 +91,10 @@ __device__ __forceinline__ float block_reduce(float v, bool is_max, float* red) 
     return v;
 }
 
-__global__ __launch_bounds__(256) void softmax_rows_kernel(const float* s, f16* p, int n, float c) {
+__global__ __launch_bounds__(256) void softmax_rows_kernel(const float* s, f16* p, int n, int ldp, float c) {
     __shared__ float red[4];
     const float* sr = s + (int64_t)blockIdx.x * n;
-    f16* pr = p + (int64_t)blockIdx.x * n;
+    f16* pr = p + (int64_t)blockIdx.x * ldp;
     float m = -INFINITY;
     for (int j = threadIdx.x; j < n; j += 256) m = fmaxf(m, sr[j]);
     m = block_reduce(m, true, red);
@@ -102,14 +102,14 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(const float* s, f16* 
     for (int j = threadIdx.x; j < n; j += 256) sum += __builtin_amdgcn_exp2f((sr[j] - m) * c);
     sum = block_reduce(sum, false, red);
     const float inv = 1.0f / sum;
-    for (int j = threadIdx.x; j < n; j += 256) pr[j] = (f16)(__builtin_amdgcn_exp2f((sr[j] - m) * c) * inv);
+    for (int j = threadIdx.x; j < ldp; j += 256) pr[j] = (f16)(j < n ? __builtin_amdgcn_exp2f((sr[j] - m) * c) * inv : 0.f);
 }
 
-hipError_t softmax_rows_launch(const float* s, f16* p, int rows, int n, float scale, hipStream_t st) {
-    if (rows < 1 || n < 1) return hipErrorInvalidValue;
+hipError_t softmax_rows_launch(const float* s, f16* p, int rows, int n, int ldp, float scale, hipStream_t st) {
+    if (rows < 1 || n < 1 || ldp < n) return hipErrorInvalidValue;
     const float c = scale * 1.4426950408889634f;
     launch_timed("softmax_rows_kernel", 0.0, (double)rows * n * 6.0, [&] {
-        SDU_LAUNCH(softmax_rows_kernel, dim3((unsigned)rows), dim3(256), 0, st, s, p, n, c);
+        SDU_LAUNCH(softmax_rows_kernel, dim3((unsigned)rows), dim3(256), 0, st, s, p, n, ldp, c);
     });
     return hipGetLastError();
 }

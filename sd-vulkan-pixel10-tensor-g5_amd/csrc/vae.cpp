@@ -245,19 +245,23 @@ static Act attention(Exec& E, AuxNet& n, Act x, int H, int W) {
         ga.bias = n.wd(a + (i ? ".to_k.bias" : ".to_q.bias"));
         gemm(E, "vae_linear", ga);
     }
-    f16* vt = E.alloc<f16>((size_t)C * HW);    // V^T of one image (to_v's bias is in to_out's)
+    // the PV product's operands have the tokens along K: rows of a multiple of 8 tokens (16-byte
+    // loads), zeros past the last one
+    const int HWp = (HW + 7) & ~7;
+    f16* vt = E.alloc<f16>((size_t)C * HWp);     // V^T of one image (to_v's bias is in to_out's)
     float* s = E.alloc<float>((size_t)HW * HW);  // scores of one image
-    f16* p = E.alloc<f16>((size_t)HW * HW);
+    f16* p = E.alloc<f16>((size_t)HW * HWp);
+    if (HWp != HW) E.run("vae_io", [&] { return zero_launch(vt, (size_t)C * HWp * sizeof(f16), E.s); });
     f16* o = E.alloc<f16>((size_t)M * C);
     const float scale = 1.0f / sqrtf((float)C);
     for (int b = 0; b < E.B; ++b) {
         const size_t t0 = (size_t)b * HW * C;
-        gemm(E, "vae_linear", dense_args(n.wd(a + ".to_v.weight"), C, C, HW, C, g + t0, vt, HW));
+        gemm(E, "vae_linear", dense_args(n.wd(a + ".to_v.weight"), C, C, HW, C, g + t0, vt, HWp));
         GemmArgs sa = dense_args(q + t0, C, HW, HW, C, k + t0, s, HW);
         sa.out_mode = OUT_F32;
         gemm(E, "vae_attn_scores", sa);
-        E.run("vae_attn_softmax", [&] { return softmax_rows_launch(s, p, HW, HW, scale, E.s); });
-        gemm(E, "vae_attn_pv", dense_args(p, HW, HW, C, HW, vt, o + t0, C));
+        E.run("vae_attn_softmax", [&] { return softmax_rows_launch(s, p, HW, HW, HWp, scale, E.s); });
+        gemm(E, "vae_attn_pv", dense_args(p, HWp, HW, C, HWp, vt, o + t0, C));
     }
     GemmArgs oa = dense_args(o, C, M, C, C, n.wd(a + ".to_out.0.weight"), out, C);
     oa.bias2 = n.b_attn_out;

@@ -40,6 +40,10 @@ def vae_weights():
     (2, 8, 12),    # two images, a non-square latent
     (1, 16, 16),   # epilogue statistics from 64x64 pixels up
     (1, 64, 64),   # the reference's contract: [1,4,64,64] -> [1,3,512,512]
+    # the mid block's attention over a token count that is no multiple of 8
+    (1, 9, 11),    # 99 tokens
+    (2, 13, 9),    # 117, two images
+    (1, 51, 37),   # 1887
 ])
 def test_vae_decode_matches_oracle(vae_engine, vae_weights, B, H, W):
     say(f"vae decode B={B} {H}x{W}")
