@@ -4,13 +4,10 @@
 // [1, 77, 768], the UNet's cross-attention context), an export of SD1.5's text_encoder
 // (CLIP ViT-L/14 text tower: 12 pre-LayerNorm layers of width 768, 12 heads, quick-GELU MLP
 // of 3072, causal self-attention, final LayerNorm).  Per layer:
-//   qkv = LN1(x) Wqkv^T + b                     (one GEMM over the fused q/k/v weight)
-//   x += out_proj(causal_attention(q, k, v))
-//   x += fc2(quick_gelu(fc1(LN2(x))))           (quick-GELU in fc1's epilogue)
-// with the residual adds in the GEMM epilogues (in place on x), activations fp16.  LN1 and LN2
-// run inside the GEMMs around them: the one that writes x keeps its row statistics, the one
-// that reads it has the affine folded into its weight (as separate launches they took 113 of
-// 554 us for two prompts).
+//   h = LN1(x); qkv = h Wqkv^T + b (one GEMM over the fused q/k/v weight);
+//   x += out_proj(causal_attention(q, k, v));  h = LN2(x);
+//   x += fc2(quick_gelu(fc1(h)))                (quick-GELU in fc1's epilogue)
+// with the residual adds in the GEMM epilogues (in place on x), activations fp16.
 #include "graph.h"
 
 namespace sdu {
@@ -52,32 +49,14 @@ int clip_create(Ctx& c, const char* weights_dir, uint64_t seed, int flags) {
     AuxNet* n = new AuxNet();
     n->kind = AUX_CLIP;
     clip_register(*n);
-    // folded projections, each [N, C] weight, then [N] bias and [N] column sums (fp32)
-    const int lnN[2] = {3 * kHid, kFfn};
-    const auto fold_bytes = [](int N) { return (size_t)N * (kHid * sizeof(f16) + 2 * sizeof(float)); };
-    const size_t extra = kLayers * (fold_bytes(lnN[0]) + fold_bytes(lnN[1]));
-    int st = aux_alloc(c, *n, extra);
+    int st = aux_alloc(c, *n, 0);
     if (st) { aux_free(n); return st; }
     const bool affine = (flags & SDU_INIT_RANDOM_AFFINE) != 0;
     for (const WeightRec& r : n->weights) {
         st = weights_dir ? load_weight_file(c, r, weights_dir) : gen_weight(c, r, seed, affine, 0.02);
         if (st) { aux_free(n); return st; }
     }
-    char* p = (char*)n->pool + n->pool_bytes - extra;
-    hipError_t e = hipSuccess;
-    for (int i = 0; i < 2 * kLayers && e == hipSuccess; ++i) {
-        const std::string pf = layer(i / 2), w = i % 2 ? ".mlp.fc1" : ".self_attn.q_proj", g = i % 2 ? ".layer_norm2" : ".layer_norm1";
-        const int N = lnN[i % 2];
-        AuxNet::LnLinear l;
-        l.w = (f16*)p;
-        l.b = (float*)(l.w + (size_t)N * kHid);
-        l.s = l.b + N;
-        p += fold_bytes(N);
-        n->ln.push_back(l);
-        e = fold_ln_launch(n->wd(pf + w + ".weight"), n->wd(pf + w + ".bias"), n->wd(pf + g + ".weight"), n->wd(pf + g + ".bias"),
-                           l.w, l.b, l.s, N, kHid, c.stream);
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    hipError_t e = hipStreamSynchronize(c.stream);
     if (e != hipSuccess) { aux_free(n); return hip_fail(c, e, "clip weights"); }
     aux_free(c.clip);
     c.clip = n;
@@ -91,25 +70,23 @@ static void clip_body(Exec& E, AuxNet& n, AuxState& S) {
     f16* qkv = E.alloc<f16>((size_t)T * 3 * C);
     f16* at = E.alloc<f16>((size_t)T * C);
     f16* f = E.alloc<f16>((size_t)T * kFfn);
-    // row statistics of x before each layer's LayerNorms (GemmArgs::row_part)
-    float* rp1 = E.alloc<float>((size_t)(C / 64) * T * 2);
-    float* rp2 = E.alloc<float>((size_t)(C / 64) * T * 2);
     E.run("clip_embed", [&] {
         return embed_launch((const int32_t*)S.in, n.wd(kPf + "embeddings.token_embedding.weight"),
-                            n.wd(kPf + "embeddings.position_embedding.weight"), x, rp1, B, kSeq, C, kVocab, E.s);
+                            n.wd(kPf + "embeddings.position_embedding.weight"), x, B, kSeq, C, kVocab, E.s);
     });
-    // a projection of LayerNorm(x), the LayerNorm inside the GEMM
-    auto ln_gemm = [&](const AuxNet::LnLinear& l, int N, const float* part, f16* out) {
-        GemmArgs g = dense_args(x, C, T, N, C, l.w, out, N);
-        g.bias2 = l.b;
-        g.ln_part = part;
-        g.ln_colsum = l.s;
-        g.ln_eps = kLnEps;
-        return g;
+    auto ln = [&](const f16* in, const std::string& pf, f16* out) {
+        E.run("clip_ln", [&] {
+            return layernorm_launch(in, n.wd(pf + ".weight"), n.wd(pf + ".bias"), out, T, C, kLnEps, E.s);
+        });
     };
     for (int i = 0; i < kLayers; ++i) {
         const std::string pf = layer(i), a = pf + ".self_attn.";
-        gemm(E, "clip_linear", ln_gemm(n.ln[2 * i], 3 * C, rp1, qkv));
+        ln(x, pf + ".layer_norm1", h);
+        {
+            GemmArgs g = dense_args(h, C, T, 3 * C, C, n.wd(a + "q_proj.weight"), qkv, 3 * C);
+            g.bias = n.wd(a + "q_proj.bias");
+            gemm(E, "clip_linear", g);
+        }
         AttnArgs aa{qkv, qkv + C, qkv + 2 * C, at, B, kHeads, kSeq, kSeq, C / kHeads, 3 * C, 3 * C, 3 * C, C,
                     1.0f / sqrtf((float)(C / kHeads)), 1};
         E.run("clip_attn", [&] { return attention_launch(aa, E.s); });
@@ -118,11 +95,12 @@ static void clip_body(Exec& E, AuxNet& n, AuxState& S) {
             g.bias = n.wd(a + "out_proj.bias");
             g.res = x;
             g.ldr = C;
-            g.row_part = rp2;
             gemm(E, "clip_linear", g);
         }
+        ln(x, pf + ".layer_norm2", h);
         {
-            GemmArgs g = ln_gemm(n.ln[2 * i + 1], kFfn, rp2, f);
+            GemmArgs g = dense_args(h, C, T, kFfn, C, n.wd(pf + ".mlp.fc1.weight"), f, kFfn);
+            g.bias = n.wd(pf + ".mlp.fc1.bias");
             g.act = ACT_QUICK_GELU;
             gemm(E, "clip_linear", g);
         }
@@ -131,13 +109,10 @@ static void clip_body(Exec& E, AuxNet& n, AuxState& S) {
             g.bias = n.wd(pf + ".mlp.fc2.bias");
             g.res = x;
             g.ldr = C;
-            g.row_part = rp1;
             gemm(E, "clip_linear", g);
         }
     }
-    E.run("clip_ln", [&] {
-        return layernorm_launch(x, n.wd(kPf + "final_layer_norm.weight"), n.wd(kPf + "final_layer_norm.bias"), h, T, C, kLnEps, E.s);
-    });
+    ln(x, kPf + "final_layer_norm", h);
     E.run("clip_io", [&] { return f16_to_f32_launch(h, (float*)S.out, (int64_t)T * C, E.s); });
 }
 

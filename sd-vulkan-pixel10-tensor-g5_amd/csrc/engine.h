@@ -119,13 +119,6 @@ struct AuxNet {
     f16* w2sc[2] = {nullptr, nullptr};
     f16* b2sc[2] = {nullptr, nullptr};
     float* b_attn_out = nullptr;
-    // CLIP: each layer's q/k/v and fc1 projections with the LayerNorm before them folded in
-    // (fold_ln_launch): weight, bias, column sums
-    struct LnLinear {
-        f16* w;
-        float *b, *s;
-    };
-    std::vector<LnLinear> ln;
     // VAE / TAESD: sub-pixel weights of the convs after each 2x upsampling (GemmArgs::subpix)
     f16* w4[3] = {nullptr, nullptr, nullptr};
     int add(const std::string& name, std::vector<int64_t> shape, int kind, int layout = GL_PLAIN, int ci_pad = 0,

@@ -511,7 +511,7 @@ bool dense_ok(const GemmArgs& a) {
     if (256LL * a.ldc * (a.out_mode == OUT_F32 ? 4 : 2) > 1 << 30 || (a.res && 256LL * a.ldr * 2 > 1 << 30)) return false;
     if (a.geglu) return !a.res && !a.act && a.out_mode == OUT_F16;
     if (a.ln_part || a.row_part || a.stats)
-        return (!a.act || (a.ln_part && a.act == ACT_QUICK_GELU)) && a.out_mode == OUT_F16 && !(a.row_part && a.stats) &&
+        return !a.act && a.out_mode == OUT_F16 && !(a.row_part && a.stats) &&
                (a.ln_part ? !a.res && !a.row_part && !a.stats : !a.stats || a.stats_hw % 16 == 0);
     if (a.out_mode == OUT_F32 || a.act) return !a.res && a.out_mode != OUT_F32_NCHW && (a.out_mode == OUT_F16 ? a.act == ACT_QUICK_GELU : !a.act);
     return a.out_mode == OUT_F16;
@@ -531,7 +531,6 @@ static void launch(dim3 grid, dim3 blk, const GemmArgs& a, hipStream_t s) {
         case 2 * EP_GEGLU: SDU_LAUNCH((gemm_dense_kernel<MT, NT, WM, WN, NS, WPE, false, EP_GEGLU>), grid, blk, 0, s, a); break;
         case 2 * EP_GEGLU + 1: SDU_LAUNCH((gemm_dense_kernel<MT, NT, WM, WN, NS, WPE, true, EP_GEGLU>), grid, blk, 0, s, a); break;
         case 2 * EP_QGELU: SDU_LAUNCH((gemm_dense_kernel<MT, NT, WM, WN, NS, WPE, false, EP_QGELU>), grid, blk, 0, s, a); break;
-        case 2 * EP_QGELU + 1: SDU_LAUNCH((gemm_dense_kernel<MT, NT, WM, WN, NS, WPE, true, EP_QGELU>), grid, blk, 0, s, a); break;
         case 2 * EP_F32: SDU_LAUNCH((gemm_dense_kernel<MT, NT, WM, WN, NS, WPE, false, EP_F32>), grid, blk, 0, s, a); break;
     }
 }

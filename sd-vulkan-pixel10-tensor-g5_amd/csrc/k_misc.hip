@@ -158,10 +158,9 @@ hipError_t stage_in_launch(const float* lat, const float* ctx, const float* temb
     return hipGetLastError();
 }
 
-// One thread per 8 channels of one token; row_part: the row statistics of the output, as a GEMM's
-// (GemmArgs::row_part), from the 8 consecutive lanes of each 64 channels.
-__global__ void embed_kernel(const int32_t* ids, const f16* tok, const f16* pos, f16* out, float* row_part, int B, int S,
-                             int C, int vocab) {
+// One thread per 8 channels of one token.
+__global__ void embed_kernel(const int32_t* ids, const f16* tok, const f16* pos, f16* out, int B, int S, int C,
+                             int vocab) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int cpr = C / 8;
     if (i >= (int64_t)B * S * cpr) return;
@@ -178,28 +177,15 @@ __global__ void embed_kernel(const int32_t* ids, const f16* tok, const f16* pos,
 #pragma unroll
     for (int e = 0; e < 8; ++e) oh[e] = (f16)((float)ah[e] + (float)ph[e]);
     *(uint4*)(out + row * C + c8) = o;
-    float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float f = (float)oh[e];
-        s1 += f;
-        s2 += f * f;
-    }
-#pragma unroll
-    for (int off = 1; off < 8; off <<= 1) {
-        s1 += __shfl_xor(s1, off);
-        s2 += __shfl_xor(s2, off);
-    }
-    if ((c8 & 63) == 0) *(float2*)(row_part + ((int64_t)(c8 >> 6) * B * S + row) * 2) = make_float2(s1, s2);
 }
 
-hipError_t embed_launch(const int32_t* ids, const f16* tok, const f16* pos, f16* out, float* row_part, int B, int S,
-                        int C, int vocab, hipStream_t s) {
-    if (B < 1 || S < 1 || C % 64 || vocab < 1) return hipErrorInvalidValue;
+hipError_t embed_launch(const int32_t* ids, const f16* tok, const f16* pos, f16* out, int B, int S, int C,
+                        int vocab, hipStream_t s) {
+    if (B < 1 || S < 1 || C % 8 || vocab < 1) return hipErrorInvalidValue;
     const int64_t total = (int64_t)B * S * (C / 8);
     launch_timed("embed_kernel", 0.0, 4.0 * B * S * C + 4.0 * B * S, [&] {
-        SDU_LAUNCH(embed_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, ids, tok, pos, out, row_part,
-                   B, S, C, vocab);
+        SDU_LAUNCH(embed_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, ids, tok, pos, out, B, S, C,
+                   vocab);
     });
     return hipGetLastError();
 }

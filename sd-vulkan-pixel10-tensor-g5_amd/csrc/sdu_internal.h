@@ -249,10 +249,9 @@ hipError_t stage_in_launch(const float* lat, const float* ctx, const float* temb
                            hipStream_t s, void* zero_dst = nullptr, size_t zero_bytes = 0,
                            void** out_slot = nullptr, void* out_ptr = nullptr);
 // Token + position embedding: out[b*S + i][:] = tok[ids[b*S + i]][:] + pos[i][:] (fp16,
-// summed in fp32), ids clamped to [0, vocab); row_part: its row statistics (GemmArgs::row_part).
-// C % 64 == 0.
-hipError_t embed_launch(const int32_t* ids, const f16* tok, const f16* pos, f16* out, float* row_part, int B, int S,
-                        int C, int vocab, hipStream_t s);
+// summed in fp32), ids clamped to [0, vocab).  C % 8 == 0.
+hipError_t embed_launch(const int32_t* ids, const f16* tok, const f16* pos, f16* out, int B, int S, int C,
+                        int vocab, hipStream_t s);
 // fp32 -> fp16 copy
 hipError_t f32_to_f16_launch(const float* src, f16* dst, int64_t n, hipStream_t s);
 hipError_t f16_to_f32_launch(const f16* src, float* dst, int64_t n, hipStream_t s);
