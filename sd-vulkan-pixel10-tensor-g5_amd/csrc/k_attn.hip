@@ -21,14 +21,16 @@
 // dim tile, that row of V^T is set to 1 so the PV MFMA also produces the row sums.
 // When Q arrives pre-scaled by scale * log2 e (the UNet's query projections fold it
 // in) and the head size leaves a spare dimension in the last 16-wide k-step (d = 40),
-// the shared-tile kernel also moves the FMA into the MFMA: that dimension of Q holds
+// the shared-tile kernels also move the FMA into the MFMA: that dimension of Q holds
 // -m against a K column of ones, so the scores come out as s*c - m (ofs_update).
 //
 // Three kernels:
-//   attn_kernel       -- NWAVE query waves share each 64-key K/V tile in LDS
-//                        (long sequences: 64x64 self-attention, 4096 tokens);
-//   attn_wide_kernel  -- the same with 64 queries per wave, scores of the next keys formed
-//                        during the softmax of these (many query blocks, heads of 33..80);
+//   attn_wide_kernel  -- 4 waves of 64 queries share each 64-key K/V tile in LDS, scores of
+//                        the next keys formed during the softmax of these (heads of 33..80
+//                        with many query blocks: every level of the UNet from 32x32 up at
+//                        batch 16, its 64x64 and 96x96 self-attention at batch 2);
+//   attn_kernel       -- NWAVE waves of 32 queries share each K/V tile (other head sizes, and
+//                        grids that would give the wide kernel a short second round);
 //   attn_split_kernel -- NSPLIT waves split the keys of one 32-query group and
 //                        merge their partial (max, sum, O) through LDS (short query
 //                        counts, where one wave per 32 queries cannot fill the chip).
@@ -48,8 +50,8 @@ static constexpr float kRescaleLog2 = 8.0f;  // lazy-rescale threshold (log2 uni
 static constexpr int kAttnMaxPairs = 16384;
 // Shared-tile launches stage V row-major and read it with transposing LDS reads (TRV),
 // except with 128-key tiles: per launch, with random operands, d40 at 9216 tokens B=2
-// -4.1%, at 4096 tokens B=16 -9%, d80 -10 to -13%, d160 at B=16 -10%, but d40 with
-// 128-key tiles (4096 tokens, B=2) +1.5%
+// -4.1%, at 4096 tokens B=16 -9%, d160 at B=16 -10%, but d40 with 128-key tiles (4096
+// tokens, B=2) +1.5%
 static constexpr bool kTRV = true;
 static constexpr int kAttnCounterFloats = kAttnMaxPairs;
 
@@ -1005,8 +1007,8 @@ static int resident_blocks(Kern kern, int threads) {
     return n;
 }
 
-// How a launch runs: the shared-tile kernel (waves per block, 128-key tiles, the softmax
-// reference in a spare dimension, keys split in two) or the key-split kernel (waves per
+// How a launch runs: a shared-tile kernel (the wide one, or waves per block, 128-key tiles, keys
+// split in two; the softmax reference in a spare dimension) or the key-split kernel (waves per
 // 32-query group).
 struct AttnPlan {
     bool shared;
@@ -1020,14 +1022,6 @@ static AttnPlan attn_plan(const AttnArgs& a) {
     AttnPlan p{};
     const int64_t bh = (int64_t)a.heads * a.B;
     const int64_t qwaves = ((a.Sq + 31) / 32) * bh;  // one wave per 32 queries
-    // shared K/V tiles where there are enough query waves to fill the chip (the
-    // key-split kernel re-reads K/V per wave): four query waves per block, eight for
-    // heads of 56..128 when four would leave < 512 blocks (their larger K/V tiles are
-    // then shared by more waves; measured per shape: d80 at 2304 tokens, B=2, 0.43 ms
-    // with two waves, 0.375 with four, 0.353 with eight; d160 at 256 tokens, B=16, 0.221
-    // with two, 0.158 with four).  Fewer query waves (e.g. 1024 queries x 16 heads), and
-    // short key sequences (cross-attention over the 77 context tokens), go to the
-    // key-split kernel: its extra waves, or not staging a few K/V tiles per block, win.
     // 64 queries per wave for heads of 33..80 where their 256-query blocks cover enough of the CUs.
     // Time against the narrow tiles', d 40 / d 64: 128 blocks 0.9-1.1 / 0.8-1.0, 144 to 256
     // 0.78-0.87 / 0.81-0.98, 257 to 320 (a short second round) 1.02-1.08 / 0.78-1.05, above
@@ -1044,13 +1038,23 @@ static AttnPlan attn_plan(const AttnArgs& a) {
         p.grid = dim3((a.Sq + 255) / 256, a.heads, a.B);
         return p;
     }
-    if (qwaves >= 1024 && a.Sk > 128 && !a.causal) {
+    // Shared K/V tiles of 32 queries per wave where there are enough query waves to fill the
+    // chip (the key-split kernel re-reads K/V per wave): four query waves per block (d160 at 256
+    // tokens, B=16, 0.158 ms a forward against 0.221 with two), eight for heads of 56..128 when
+    // four would leave < 512 blocks, their larger K/V tiles then shared by more waves (1024
+    // tokens, 32 heads x images, d96 41.7 against 45.2 us, d128 50.0 against 58.6; 2304 tokens,
+    // 16: equal; d56 and d64, which come here with 128 to 143 wide blocks only, lose: 47.9
+    // against 41.1, 52.5 against 47.6).  Fewer query waves (e.g. 1024 queries x 16 heads),
+    // and short key sequences (cross-attention over the 77 context tokens), go to the
+    // key-split kernel: its extra waves, or not staging a few K/V tiles per block, win.
+    // (Heads of 65..80 with this many query waves are the wide kernel's, above.)
+    if (KS != 5 && qwaves >= 1024 && a.Sk > 128 && !a.causal) {
         p.shared = true;
         p.nw = (a.d > 48 && a.d <= 128 && ((a.Sq + 127) / 128) * bh < 512) ? 8 : 4;
         p.grid = dim3((a.Sq + p.nw * 32 - 1) / (p.nw * 32), a.heads, a.B);
-        // 128-key tiles for heads <= 48 when every block is resident at once (two per CU):
-        // d40 at 4096 tokens, B=2, 0.44 ms per forward against 0.46 with 64-key tiles;
-        // on larger grids they lose (0.24 ms more at 9216 tokens, 0.31 ms at B=16)
+        // 128-key tiles for heads <= 48 when every block is resident at once (two per CU): 260 to
+        // 300 heads x images, 128 queries, 512 keys 20.4-21.0 us against 28-29 with 64-key tiles;
+        // 16, 2048 tokens 35.6 against 36.6, but 8, 4096 tokens 64.0 against 58.8
         p.kt128 = KS == 3 && p.nw == 4 && (long)p.grid.x * bh <= 512;
         // the softmax reference rides in a spare head dimension when Q is pre-scaled
         p.ofs = a.q_log2 && a.d < KS * 16 && p.nw == 4;
@@ -1058,15 +1062,17 @@ static AttnPlan attn_plan(const AttnArgs& a) {
         // half-length blocks then fill whole rounds.  A partial last round is modelled
         // at 3/4 of a full one's time, the merge at 1/20 (d40 at 9216 tokens, B=2: 1.5
         // rounds of 768 blocks; measured 1.75 round-times)
-        if (p.nw == 4 && !p.kt128 && a.Sk > 64 && (long)p.grid.x * bh <= kAttnMaxPairs) {
-            const long nblk = (long)p.grid.x * bh;
-            const int slots = p.ofs ? resident_blocks<KS, MTD, LSUM, true>(attn_kernel<KS, MTD, 4, LSUM, 64, true, false, kTRV>, 256)
-                                    : resident_blocks<KS, MTD, LSUM, false>(attn_kernel<KS, MTD, 4, LSUM, 64, false, false, kTRV>, 256);
-            if (slots > 0) {
-                auto rounds = [&](double r) { const double f = floor(r); return f + (r > f ? 0.75 : 0.0); };
-                p.spl = rounds(2.0 * nblk / slots) * 0.5 + 0.05 < 0.9 * rounds((double)nblk / slots);
+        if constexpr (KS != 5)
+            if (p.nw == 4 && !p.kt128 && a.Sk > 64 && (long)p.grid.x * bh <= kAttnMaxPairs) {
+                const long nblk = (long)p.grid.x * bh;
+                int slots = 0;
+                if (!p.ofs) slots = resident_blocks<KS, MTD, LSUM, false>(attn_kernel<KS, MTD, 4, LSUM, 64, false, false, kTRV>, 256);
+                else if constexpr (LSUM) slots = resident_blocks<KS, MTD, LSUM, true>(attn_kernel<KS, MTD, 4, LSUM, 64, true, false, kTRV>, 256);
+                if (slots > 0) {
+                    auto rounds = [&](double r) { const double f = floor(r); return f + (r > f ? 0.75 : 0.0); };
+                    p.spl = rounds(2.0 * nblk / slots) * 0.5 + 0.05 < 0.9 * rounds((double)nblk / slots);
+                }
             }
-        }
         return p;
     }
     // key split: enough waves to fill the chip, at most one per 32-key tile, and at
@@ -1100,36 +1106,50 @@ static void launch_cfg(const AttnArgs& a0, hipStream_t s) {
         if (p.wide) {
             snprintf(name, sizeof name, "attn_wide_kernel<%d,%d,%d,%d>", KS, MTD, (int)LSUM, (int)p.ofs);
             launch_timed(name, flops, bytes, [&] {
-                if (p.ofs) SDU_LAUNCH((attn_wide_kernel<KS, MTD, LSUM, true>), p.grid, dim3(256), 0, s, a);
-                else SDU_LAUNCH((attn_wide_kernel<KS, MTD, LSUM, false>), p.grid, dim3(256), 0, s, a);
+                if constexpr (LSUM)  // (a spare dimension for the reference leaves a row for the sums, too)
+                    if (p.ofs) {
+                        SDU_LAUNCH((attn_wide_kernel<KS, MTD, LSUM, true>), p.grid, dim3(256), 0, s, a);
+                        return;
+                    }
+                SDU_LAUNCH((attn_wide_kernel<KS, MTD, LSUM, false>), p.grid, dim3(256), 0, s, a);
             });
             return;
         }
     }
-    if (p.shared) {
-        const bool spl = p.spl && a.ws;
-        const bool trv = kTRV && !p.kt128;
-        snprintf(name, sizeof name, "attn_kernel<%d,%d,%d,%d,%d,%d,%d,%d>", KS, MTD, p.nw, (int)LSUM, p.kt128 ? 128 : 64,
-                 (int)p.ofs, (int)spl, (int)trv);
-        constexpr int KTB = KS == 3 ? 128 : 64;
-        dim3 grid = p.grid;
-        if (spl) {
-            a.kpart = ((a.Sk + 127) / 128) * 64;  // half the 64-key tiles (rounded up)
-            grid.z *= 2;
+    if constexpr (KS != 5)
+        if (p.shared) {
+            const bool spl = p.spl && a.ws;
+            const bool trv = kTRV && !p.kt128;
+            snprintf(name, sizeof name, "attn_kernel<%d,%d,%d,%d,%d,%d,%d,%d>", KS, MTD, p.nw, (int)LSUM, p.kt128 ? 128 : 64,
+                     (int)p.ofs, (int)spl, (int)trv);
+            dim3 grid = p.grid;
+            if (spl) {
+                a.kpart = ((a.Sk + 127) / 128) * 64;  // half the 64-key tiles (rounded up)
+                grid.z *= 2;
+            }
+            launch_timed(name, flops, bytes, [&] {
+                if constexpr (KS == 3)
+                    if (p.kt128) {
+                        if (p.ofs) SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 128, true>), grid, dim3(256), 0, s, a);
+                        else SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 128>), grid, dim3(256), 0, s, a);
+                        return;
+                    }
+                if constexpr (LSUM)
+                    if (p.ofs) {
+                        if (spl) SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 64, true, true, kTRV>), grid, dim3(256), 0, s, a);
+                        else SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 64, true, false, kTRV>), grid, dim3(256), 0, s, a);
+                        return;
+                    }
+                if constexpr (KS >= 4 && KS <= 8)
+                    if (p.nw == 8) {
+                        SDU_LAUNCH((attn_kernel<KS, MTD, 8, LSUM, 64, false, false, kTRV>), grid, dim3(512), 0, s, a);
+                        return;
+                    }
+                if (spl) SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 64, false, true, kTRV>), grid, dim3(256), 0, s, a);
+                else SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 64, false, false, kTRV>), grid, dim3(256), 0, s, a);
+            });
+            return;
         }
-        launch_timed(name, flops, bytes, [&] {
-            if (p.nw == 8) SDU_LAUNCH((attn_kernel<KS, MTD, 8, LSUM, 64, false, false, kTRV>), grid, dim3(512), 0, s, a);
-            else if (KS == 3 && p.kt128 && p.ofs)
-                SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, KTB, true>), grid, dim3(256), 0, s, a);
-            else if (KS == 3 && p.kt128)
-                SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, KTB>), grid, dim3(256), 0, s, a);
-            else if (spl && p.ofs) SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 64, true, true, kTRV>), grid, dim3(256), 0, s, a);
-            else if (spl) SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 64, false, true, kTRV>), grid, dim3(256), 0, s, a);
-            else if (p.ofs) SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 64, true, false, kTRV>), grid, dim3(256), 0, s, a);
-            else SDU_LAUNCH((attn_kernel<KS, MTD, 4, LSUM, 64, false, false, kTRV>), grid, dim3(256), 0, s, a);
-        });
-        return;
-    }
     const int ns = p.ns;
     snprintf(name, sizeof name, "attn_split_kernel<%d,%d,%d,%d>", KS, MTD, ns, (int)LSUM);
     const dim3 grid = p.grid;
@@ -1144,13 +1164,15 @@ static void launch_cfg(const AttnArgs& a0, hipStream_t s) {
 
 template <int KS, int MTD>
 static void launch_d(const AttnArgs& a, hipStream_t s) {
-    if (a.d < MTD * 32) launch_cfg<KS, MTD, true>(a, s);
+    if constexpr (KS * 16 < MTD * 32) launch_cfg<KS, MTD, true>(a, s);
+    else if (a.d < MTD * 32) launch_cfg<KS, MTD, true>(a, s);
     else launch_cfg<KS, MTD, false>(a, s);
 }
 
 template <int KS, int MTD>
 static size_t ws_d(const AttnArgs& a) {
-    return a.d < MTD * 32 ? ws_bytes<KS, MTD, true>(a) : ws_bytes<KS, MTD, false>(a);
+    if constexpr (KS * 16 < MTD * 32) return ws_bytes<KS, MTD, true>(a);
+    else return a.d < MTD * 32 ? ws_bytes<KS, MTD, true>(a) : ws_bytes<KS, MTD, false>(a);
 }
 
 size_t attention_workspace_bytes(const AttnArgs& a) {
