@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+import tile_cases
 from conftest import rel_err_l1, say
 from oracle import lcm, unet_ref as U
 
@@ -24,6 +25,16 @@ def r16(shape, seed, scale=1.0, mean=0.0):
 
 def t(a):
     return torch.from_numpy(np.ascontiguousarray(a))
+
+
+def kernels_of(e, f):
+    """The kernels that f's op-level calls launch, by name (but for the clear of a scratch that grows)."""
+    e.profile_ops(True)
+    try:
+        f()
+    finally:
+        prof, _ = e.profile_ops(False)
+    return {n[2:] for n in prof if n.startswith("k:")} - {"zero_kernel"}
 
 
 # ------------------------------------------------------------------ GroupNorm
@@ -246,7 +257,7 @@ def test_layernorm(op_engine, T, C):
     (96, 320, 640, 0, True, True, False, True),          # ragged M, fp32 out
     (64, 1280, 1280, 0, False, True, False, False),      # M = 64
     (33, 64, 128, 0, True, False, True, False),          # ragged M, GEGLU
-    # the 64x160 tile (16x16x32 MFMAs): ragged M with split K, and the 77-token cross K/V
+    # ragged M at 320 columns, and the 77-token cross K/V
     (8000, 320, 2880, 0, True, True, False, False),
     (154, 24960, 768, 0, False, False, False, False),
     (8192, 300, 2880, 0, True, False, False, True),  # N % 8 != 0: element-wise epilogue
@@ -292,31 +303,12 @@ def test_matmul(op_engine, M, N, K, K2, bias, res, geglu, f32):
     assert np.abs(got - ref).max() < 3e-2 * max(1.0, np.abs(ref).max() / 8)
 
 
-@pytest.mark.parametrize("M,N,K,K2,bias,res,geglu,f32", [
-    (1, 8, 64, 0, True, True, False, False),          # one row, one 8-column chunk, one K step
-    (63, 72, 128, 0, True, False, False, True),       # a row short of a tile, 8 columns past one
-    (65, 64, 192, 64, False, True, False, False),     # a row past a tile, second source after 2 steps
-    (129, 136, 64, 0, True, True, False, False),
-    (257, 192, 320, 0, True, False, True, False),     # GEGLU, N not a multiple of the wide tiles
-    (40000, 136, 64, 0, True, True, False, False),    # several tiles per persistent block, one K step each
-    (33000, 320, 128, 64, True, False, False, False),  # the same, two sources of one step each
-    (20000, 640, 192, 0, True, False, True, False),   # the same, GEGLU
-    (70, 72, 2048, 0, True, True, False, False),      # split K over ragged tiles
-    (300, 200, 4096, 1024, True, True, False, False),  # split K whose later blocks start in the second source
-])
-def test_matmul_dense_tiles(op_engine, M, N, K, K2, bias, res, geglu, f32):
-    """Edges of the dense kernel's tiles and of its persistent blocks' tile hand-over."""
-    test_matmul(op_engine, M, N, K, K2, bias, res, geglu, f32)
-
-
-def kernels_of(e, f):
-    """The kernels that f's op-level calls launch, by name."""
-    e.profile_ops(True)
-    try:
-        f()
-    finally:
-        prof, _ = e.profile_ops(False)
-    return {n[2:] for n in prof if n.startswith("k:")}
+@pytest.mark.parametrize("M,N,K,K2,bias,res,geglu,f32,kernel,ksum", tile_cases.DENSE_TILES)
+def test_matmul_dense_tiles(op_engine, M, N, K, K2, bias, res, geglu, f32, kernel, ksum):
+    """Edges of the dense kernel's tiles, of its persistent blocks' tile hand-over and of its split sums."""
+    names = kernels_of(op_engine, lambda: test_matmul(op_engine, M, N, K, K2, bias, res, geglu, f32))
+    assert any(n.startswith(kernel) for n in names), names
+    assert ksum is None or ("splitk_reduce_kernel" in names) == (ksum == "reduce"), names
 
 
 @pytest.mark.parametrize("N,f32,kernel", [
@@ -401,7 +393,7 @@ def test_matmul_split_repeat(op_engine):
     (2, 16, 16, 1280, 1280, 3, 2, False, False, False),  # downsample to 8x8 (M = 128)
     (1, 8, 8, 640, 320, 3, 1, False, True, True),      # M = 64
     (1, 6, 10, 128, 96, 3, 1, False, False, True),     # ragged M = 60, Cin = 128
-    # the 64x160 tile (16x16x32 MFMAs) with split K: ragged M = 8100, non-square image
+    # 320 channels: M = 8100, non-square images
     (1, 90, 90, 320, 320, 3, 1, False, True, True),
     (2, 62, 66, 320, 320, 3, 1, False, False, False),
     (1, 90, 90, 320, 312, 3, 1, False, True, True),    # last N tile partly outside N
@@ -442,28 +434,13 @@ def test_conv2d(op_engine, B, H, W, Ci, Co, k, stride, ups, temb, res):
     assert np.abs(got - ref).max() < 3e-2
 
 
-@pytest.mark.parametrize("B,H,W,Ci,Co,temb,res", [
-    (1, 8, 8, 64, 8, False, False),        # one sub-tile of the two-sub-tile block, one chunk, N < 16
-    (3, 8, 8, 128, 72, True, True),        # odd sub-tile count, last column tile of 8
-    (1, 9, 17, 64, 168, False, True),      # one pixel past a sub-tile in both directions
-    (2, 7, 15, 192, 88, True, False),      # one pixel short
-    (1, 48, 47, 128, 128, False, True),    # a ragged column of sub-tiles
-    (1, 256, 256, 64, 136, False, False),  # 16x16 sub-tiles, last column tile of 8
-    (5, 64, 64, 320, 320, True, True),     # 160-column tiles
-    (1, 250, 243, 128, 128, True, False),  # 16x16 sub-tiles, both directions ragged
-    (2, 8, 8, 1280, 1280, False, True),    # split K with the reduce launch
-    (1, 16, 16, 704, 320, True, False),    # 11 chunks over uneven splits
-    (2, 36, 28, 640, 640, True, True),     # all taps' weights in the ring: 10 chunks
-    (1, 33, 39, 64, 72, False, True),      # one sub-tile x 32 columns, one chunk, ragged
-    (1, 128, 120, 64, 64, True, True),     # one sub-tile x 64 columns
-    (1, 16, 16, 1280, 1280, True, True),   # small tiles, split K
-    (1, 256, 250, 64, 64, True, True),     # one chunk: two 16x16 tiles per CU, a ragged column
-    (3, 203, 190, 64, 72, False, False),   # the same, both directions and the columns ragged
-])
-def test_conv_patch_tiles(op_engine, B, H, W, Ci, Co, temb, res):
-    """Edges of the patch-resident 3x3 kernel's tiles: 8x8 and 16x16 sub-tiles of ragged
-    images, column tiles of 64, 80, 128 and 160, split K at chunk boundaries."""
-    test_conv2d(op_engine, B, H, W, Ci, Co, 3, 1, False, temb, res)
+@pytest.mark.parametrize("B,H,W,Ci,Co,temb,res,kernel,ksum", tile_cases.CONV)
+def test_conv_patch_tiles(op_engine, B, H, W, Ci, Co, temb, res, kernel, ksum):
+    """Edges of the patch-resident 3x3 kernel's tiles: every shape of it on ragged images and columns, K
+    whole and split at chunk boundaries, summed in the kernel and by the reduce launch."""
+    names = kernels_of(op_engine, lambda: test_conv2d(op_engine, B, H, W, Ci, Co, 3, 1, False, temb, res))
+    assert kernel in names, names
+    assert ("splitk_reduce_kernel" in names) == (ksum == "reduce"), names
 
 
 @pytest.mark.parametrize("M,N,K", [
@@ -550,7 +527,7 @@ def test_conv2d_inplace_residual_and_overlap_errors(op_engine):
     (2, 8, 4096, 4096, 40),   # level-0 self-attention
     (2, 8, 4096, 77, 40),     # level-0 cross-attention
     (2, 8, 1024, 1024, 80),
-    (2, 8, 2304, 2304, 80),   # 96x96 level-1 self-attention: eight query waves per block
+    (2, 8, 2304, 2304, 80),   # 96x96 level-1 self-attention
     (16, 8, 256, 256, 160),   # B=16 level-2 self-attention: shared K/V tiles, four waves
     (2, 8, 256, 256, 160),
     (2, 8, 64, 64, 160),      # mid block
@@ -563,17 +540,15 @@ def test_conv2d_inplace_residual_and_overlap_errors(op_engine):
     (1, 1, 33, 65, 56),
     (1, 2, 40, 50, 96),
     (1, 1, 20, 30, 120),
-    # the shared-tile kernel with ragged query and key counts (a last query block with
-    # 2 valid queries; last key tiles with 6, 13 and 60 valid keys)
-    (2, 8, 2050, 1030, 40),   # 128-key tiles (at most 512 blocks)
-    (4, 8, 4000, 333, 40),    # 64-key tiles
-    (4, 8, 1000, 700, 80),    # eight query waves per block
-    # many shared-tile blocks (more than one round): ragged query count (last block with
-    # 4 queries) and key count (last 64-key tile with 13)
+    # ragged query and key counts (a last query block with 2 valid queries; last key tiles
+    # with 6, 13 and 60 valid keys)
+    (2, 8, 2050, 1030, 40),
+    (4, 8, 4000, 333, 40),
+    (4, 8, 1000, 700, 80),
+    # more than one round of blocks: ragged query count (last block with 4 queries) and key
+    # count (last 64-key tile with 13)
     (8, 8, 4100, 333, 40),
     (4, 16, 2048, 200, 40),
-    # keys split in two halves merged in-kernel (1.33 and 1.5 rounds of blocks; half a
-    # round, with a ragged key count: halves of 1024 and 976 keys)
     (2, 8, 9216, 9216, 40),   # UNet 96x96 self-attention
     (3, 8, 2000, 1000, 40),
 ])
@@ -617,16 +592,15 @@ def test_attention_strided_rows(op_engine):
 # Heads whose size leaves a spare MFMA dimension (8, 24, 40, 56) on the shared-tile kernel
 # carry the softmax reference in that dimension; the others only drop the scale.
 @pytest.mark.parametrize("B,heads,Sq,Sk,d", [
-    (2, 8, 4096, 4096, 40),   # UNet 64x64 self-attention: 128-key tiles
+    (2, 8, 4096, 4096, 40),   # UNet 64x64 self-attention
     (2, 8, 2050, 1030, 40),   # ragged: last query block 2 queries, last key tile 6 keys
-    (8, 8, 4100, 333, 40),    # 64-key tiles, more than one round of blocks
+    (8, 8, 4100, 333, 40),    # more than one round of blocks
     (4, 8, 1100, 300, 24),    # reference dimension in the second k-step
     (4, 8, 1100, 300, 8),     # reference dimension in the first k-step
     (8, 8, 2048, 300, 56),    # four k-steps, dimension 56
     (1, 2, 100, 37, 40),      # key-split kernel (no reference dimension)
-    (4, 8, 1000, 700, 80),    # eight-wave shared tiles (d a multiple of 16)
+    (4, 8, 1000, 700, 80),    # d a multiple of 16: no spare dimension
     (2, 8, 256, 256, 160),
-    # keys split in two halves merged in-kernel, with the reference dimension
     (2, 8, 9216, 9216, 40),   # UNet 96x96 self-attention
     (3, 8, 2000, 1000, 40),
     (4, 16, 2048, 200, 40),
@@ -652,7 +626,7 @@ def test_attention_q_log2(op_engine, B, heads, Sq, Sk, d):
     np.testing.assert_array_equal(to.numpy().astype(np.float32), got)
 
 
-@pytest.mark.parametrize("B", [4, 16])  # 128-key tiles (256 blocks), 64-key tiles (1024)
+@pytest.mark.parametrize("B", [4, 10, 16])  # 128-key tiles, 64-key tiles, 64 queries per wave
 def test_attention_q_log2_reference_moves(op_engine, B):
     """Score offsets per key range (log2 units) that move the softmax reference carried in
     the spare head dimension: the first tile far below zero (-3000), the next 10 higher
@@ -698,8 +672,42 @@ def test_attention_q_log2_reference_moves(op_engine, B):
 ])
 def test_attention_wide(op_engine, B, heads, Sq, Sk, d):
     """Edges of the 64-queries-per-wave kernel's query blocks and key steps, with either form of the scale."""
-    test_attention(op_engine, B, heads, Sq, Sk, d)
-    test_attention_q_log2(op_engine, B, heads, Sq, Sk, d)
+    names = kernels_of(op_engine, lambda: test_attention(op_engine, B, heads, Sq, Sk, d))
+    names |= kernels_of(op_engine, lambda: test_attention_q_log2(op_engine, B, heads, Sq, Sk, d))
+    assert all(n.startswith("attn_wide_kernel") for n in names), names
+
+
+# kernel: attn_kernel<k-steps, dim tiles, waves, row sums in the MFMA, keys per tile, reference in a spare
+# dimension, keys split in two, transposing V reads>, with the scale in the softmax; ofs: with q
+# pre-scaled the reference rides in the spare dimension
+@pytest.mark.parametrize("B,heads,Sq,Sk,d,kernel,ofs", [
+    (2, 8, 2046, 1030, 40, "3,2,4,1,128,0,0,0", 1),  # a query block short of 2; a last key tile of 6
+    (1, 260, 97, 131, 48, "3,2,4,1,128,0,0,0", 0),
+    (5, 8, 2000, 333, 40, "3,2,4,1,64,0,0,1", 1),
+    (5, 8, 2000, 333, 48, "3,2,4,1,64,0,0,1", 0),
+    (2, 8, 2040, 301, 56, "4,2,8,1,64,0,0,1", 0),    # eight waves carry no reference
+    (2, 8, 2040, 301, 64, "4,2,8,0,64,0,0,1", 0),
+    (9, 8, 1000, 300, 56, "4,2,4,1,64,0,0,1", 1),
+    (4, 8, 2400, 300, 64, "4,2,4,0,64,0,1,1", 0),
+    (4, 8, 1100, 200, 24, "2,1,4,1,64,0,1,1", 1),
+    (8, 8, 1100, 200, 24, "2,1,4,1,64,0,0,1", 1),
+    (8, 8, 1100, 200, 32, "2,1,4,0,64,0,0,1", 0),
+    (4, 8, 1100, 200, 88, "6,3,8,1,64,0,0,1", 0),
+    (16, 8, 1100, 200, 88, "6,3,4,1,64,0,1,1", 1),
+    (8, 8, 1100, 200, 96, "6,3,4,0,64,0,1,1", 0),
+    (12, 8, 1100, 200, 104, "8,4,4,1,64,0,0,1", 1),
+    (8, 8, 1100, 200, 128, "8,4,4,0,64,0,1,1", 0),
+    (4, 8, 1100, 200, 136, "10,5,4,1,64,0,1,1", 1),
+    (12, 8, 1100, 200, 160, "10,5,4,0,64,0,0,1", 0),
+])
+def test_attention_narrow_tiles(op_engine, B, heads, Sq, Sk, d, kernel, ofs):
+    """Each form of the 32-queries-per-wave shared-tile kernel, ragged in queries and keys."""
+    names = kernels_of(op_engine, lambda: test_attention(op_engine, B, heads, Sq, Sk, d))
+    assert names == {f"attn_kernel<{kernel}>"}
+    names = kernels_of(op_engine, lambda: test_attention_q_log2(op_engine, B, heads, Sq, Sk, d))
+    f = kernel.split(",")
+    f[5] = str(ofs)
+    assert names == {f"attn_kernel<{','.join(f)}>"}
 
 
 def test_split_ops_share_scratch(op_engine):
@@ -708,9 +716,11 @@ def test_split_ops_share_scratch(op_engine):
     for _ in range(2):
         test_matmul(op_engine, 70, 72, 2048, 0, True, True, False, False)
         test_groupnorm(op_engine, 2, 64, 64, 640, 320, True)
-        test_attention_q_log2(op_engine, 5, 8, 1800, 300, 56)  # keys split in two
+        names = kernels_of(op_engine, lambda: test_attention_q_log2(op_engine, 4, 8, 1100, 300, 24))
+        assert names == {"attn_kernel<2,1,4,1,64,1,1,1>"}  # keys split in two
         test_conv_groupnorm_epilogue_stats(op_engine, 2, 8, 8, 1280, 1280, 0.0, True, False, True)
-        test_conv_patch_tiles(op_engine, 2, 8, 8, 1280, 1280, False, True)
+        test_conv2d(op_engine, 2, 8, 8, 1280, 1280, 3, 1, False, False, True)  # summed in the kernel
+        test_conv2d(op_engine, 2, 16, 16, 1280, 1280, 3, 1, False, False, True)  # with the reduce launch
 
 
 # ------------------------------------------------------------------ elementwise
