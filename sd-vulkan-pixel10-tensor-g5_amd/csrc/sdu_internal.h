@@ -97,9 +97,9 @@ struct GemmArgs {
     // Wo = 2 Win, Cin % 64 == 0): output pixel (2y + py, 2x + px) only sees input rows
     // y + py - 1 + {0, 1} and columns x + px - 1 + {0, 1}, so each of the four phases
     // (py, px) is a 2x2 conv of the input with summed taps (fold_subpix_launch): Wt is
-    // [4 phases][N][4 taps * Cin], K = 4 Cin, and GEMM row m = phase * (M / 4) + input
-    // pixel, stored at its output pixel.  M / 4 must be a multiple of the tile rows
-    // (the planner's choice); no residual, fp16 output, no split-K reduce launch.
+    // [4 phases][N][4 taps * Cin], K = 4 Cin, and each tile is one phase's, stored at its
+    // output pixels (conv3_patch_kernel alone; any image size).  No residual, fp16 output,
+    // no split-K reduce launch.
     int subpix;
     // B operand: W [N, K] row-major
     const f16* Wt;

@@ -115,7 +115,8 @@ int taesd_create(Ctx& c, const char* weights_dir, uint64_t seed, int flags) {
 static void conv(Exec& E, const f16* x, int B, int h, int w, int cin, int ups, const f16* W, const f16* bias,
                  const f16* res, f16* y, const f16* w4 = nullptr) {
     GemmArgs a = conv3_args(x, B, h, w, cin, kCh, 1, ups, W, y);
-    // after the 2x upsampling: the sub-pixel form where each phase's pixels fill whole tiles
+    // after the 2x upsampling: the sub-pixel form for pixel counts in 64s (the kernel takes any;
+    // the others keep the 9-tap form, whose sums round differently)
     if (ups && w4 && (B * h * w) % 64 == 0) {
         a.upsample = 0;
         a.subpix = 1;

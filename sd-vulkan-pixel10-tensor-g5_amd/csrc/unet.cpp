@@ -181,7 +181,8 @@ static Act conv3_block(Exec& E, const std::string& pf, const f16* x, int H, int 
                        int stride, int ups) {
     GemmArgs a = conv3_args(x, E.B, H, Wd, Cin, Cout, stride, ups, W(E, pf + ".weight"), nullptr);
     // after a 2x nearest upsampling: the sub-pixel form (4 taps per output pixel instead of 9)
-    // where each phase's input pixels fill whole tiles
+    // for pixel counts in 64s (the kernel takes any; the others keep the 9-tap form, whose
+    // sums round differently)
     if (ups && Cin % 64 == 0 && (E.B * H * Wd) % 64 == 0)
         for (const UpDesc& u : E.c.ups)
             if (u.pf == pf && u.c == Cin && Cout == Cin) {

@@ -183,7 +183,8 @@ static f16* conv(Exec& E, AuxNet& n, const std::string& pf, Act x, int H, int W,
     const int Ho = ups ? 2 * H : H, Wo = ups ? 2 * W : W;
     f16* y = E.alloc<f16>((size_t)E.B * Ho * Wo * cout);
     GemmArgs a = conv3_args(x.p, E.B, H, W, cin, cout, 1, ups, n.wd(pf + ".weight"), y);
-    // after the 2x upsampling: the sub-pixel form where each phase's pixels fill whole tiles
+    // after the 2x upsampling: the sub-pixel form for pixel counts in 64s (the kernel takes any;
+    // the others keep the 9-tap form, whose sums round differently)
     if (ups && w4 && cin % 64 == 0 && (E.B * H * W) % 64 == 0) {
         a.upsample = 0;
         a.subpix = 1;
