@@ -1,4 +1,4 @@
-// Device helpers shared by the MFMA kernels (k_gemm.hip, k_conv.hip).
+// Device helpers shared by the MFMA kernels (k_gemm.hip, k_conv.hip, k_dense.hip).
 #pragma once
 
 #include "sdu_internal.h"

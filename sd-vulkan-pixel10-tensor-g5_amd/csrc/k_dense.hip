@@ -11,7 +11,7 @@
 // 1.14 PFLOP/s, 303 us in gemm_kernel), by the epilogue and its bytes at small K
 // (65536 x 2560 x 320 GEGLU 150 us against 221, 65536 x 320 x 320 30 against 37, 16384 x 5120 x
 // 640 GEGLU 128 against 172), by one block's latency chain where the shape has few tiles
-// (154 x 768 x 768 8.7 against 11.5).  What gave it: the epilogue in registers (no LDS round trip
+// (154 x 768 x 768 8.7 against 11.5, a clear launch in both; 7.2 without it).  What gave it: the epilogue in registers (no LDS round trip
 // of the tile), the DMA running on across a tile's epilogue, and LDS reads placed among the
 // MFMAs.  A 128 x 160 tile spilled and won one shape (16384 x 640 x 3200); rings of 4 to 9
 // stages at one block per CU lost 10-30% on operands that come from HBM.

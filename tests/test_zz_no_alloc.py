@@ -40,8 +40,8 @@ def _case(e, B, H, W, C1, C2, silu, seed):
 def test_groupnorm_noalloc_matches_groupnorm(op_engine):
     import sdu
     e = op_engine
-    # large slabs (the chunked statistics pass that accumulates into the scratch), then a
-    # smaller call on the same device: the scratch must be cleared, not reused
+    # large slabs (the statistics pass, whose partials are in the scratch), then smaller calls on
+    # the same device: each must read only what it wrote itself
     for (B, H, W, C1, C2, silu, seed) in ((4, 64, 64, 640, 320, True, 1), (1, 64, 64, 320, 0, False, 2),
                                           (2, 8, 8, 1280, 0, True, 3)):
         say(f"groupnorm_noalloc B={B} {H}x{W} C1={C1} C2={C2} silu={silu}")
