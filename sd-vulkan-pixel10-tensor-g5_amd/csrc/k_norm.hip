@@ -67,7 +67,7 @@ __device__ __forceinline__ GnSrc gn_src(const f16* x, const f16* x2, int C1, int
 // of groups whose mean dwarfs their spread, and fp32 ones less a value of the group that of groups
 // where that value is an outlier (relative error 1e-3 at 300 spreads); the conversions are no more
 // instructions than the shift was.  8 pixels per thread and round, all in flight.  Bound by latency
-// at the networks' sizes: 2 x 4096 x 960 with its apply 16.8 us (17.3 to 17.6 with shifted fp32 sums,
+// at the networks' sizes: 2 x 4096 x 960 with its apply 17.0 us (17.3 to 17.6 with shifted fp32 sums,
 // whose shift was one more dependent load; 37.1 with fp64 atomics per 8192 elements and their clear).
 __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, const f16* x2, int C1, int C2, int HW,
                                                               int P, int G, float2* part) {
@@ -76,7 +76,9 @@ __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, cons
     const int b = blockIdx.y, tid = threadIdx.x;
     const int ph = tid / V, o = tid - ph * V;
     const int p0 = blockIdx.x * P, pe = min(HW, p0 + P);
-    __shared__ __attribute__((aligned(16))) double s1[GN_THREADS * 8], s2[GN_THREADS * 8];  // [R][C]
+    // [R][C], rows of C + 2: a group's reads of consecutive rows fall on other banks
+    const int S = C + 2;
+    __shared__ __attribute__((aligned(16))) double s1[GN_THREADS * 10], s2[GN_THREADS * 10];
     if (ph < R) {
         const GnSrc src = gn_src(x, x2, C1, C2, o * 8);
         const f16* base = src.p + (int64_t)b * HW * src.ld;
@@ -99,8 +101,8 @@ __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, cons
                     q[e] = fma(f, f, q[e]);
                 }
         }
-        double2* w1 = (double2*)(s1 + ph * C + o * 8);
-        double2* w2 = (double2*)(s2 + ph * C + o * 8);
+        double2* w1 = (double2*)(s1 + ph * S + o * 8);
+        double2* w2 = (double2*)(s2 + ph * S + o * 8);
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
             w1[e / 2] = make_double2(a[e], a[e + 1]);
@@ -108,22 +110,31 @@ __global__ __launch_bounds__(GN_THREADS) void gn_stats_kernel(const f16* x, cons
         }
     }
     __syncthreads();
-    // 16 threads per group
-    const int g = tid / 16;
+    // TPG threads (at most a wave) per group, its R cpg sums dealt over them: with 16 threads that
+    // each walked the R rows of their channels, few channels left most of them idle in front of up
+    // to 512 dependent adds (2 x 112 x 32 18.7 us with the apply, 2 x 13 x 8 in 8 groups 48.7; 8.7
+    // and 8.0 so)
+    const int TPG = G > 16 ? 16 : G > 8 ? 32 : 64;
+    const int g = tid / TPG, sub = tid % TPG;
     if (g >= G) return;
     double ga = 0.0, gq = 0.0;
-    for (int r = 0; r < R; ++r)
-        for (int i = tid % 16; i < cpg; i += 16) {
-            ga += s1[r * C + g * cpg + i];
-            gq += s2[r * C + g * cpg + i];
-        }
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
+    const int dr = TPG / cpg, di = TPG - dr * cpg;
+    int r = sub / cpg, i = sub - r * cpg;
+#pragma unroll 4
+    for (int k = sub; k < R * cpg; k += TPG) {
+        const int at = r * S + g * cpg + i;
+        ga += s1[at];
+        gq += s2[at];
+        r += dr;
+        i += di;
+        if (i >= cpg) { i -= cpg; ++r; }
+    }
+    for (int off = 1; off < TPG; off <<= 1) {
         ga += __shfl_xor(ga, off);
         gq += __shfl_xor(gq, off);
     }
     const double mean = ga / ((double)(pe - p0) * cpg);
-    if (tid % 16 == 0) part[((int64_t)b * gridDim.x + blockIdx.x) * G + g] = make_float2((float)mean, (float)(gq - ga * mean));
+    if (sub == 0) part[((int64_t)b * gridDim.x + blockIdx.x) * G + g] = make_float2((float)mean, (float)(gq - ga * mean));
 }
 
 // (v_rcp_f32 is within 1 ulp: an error of 2^-24 in front of the fp16 rounding)

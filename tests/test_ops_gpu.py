@@ -87,6 +87,33 @@ def test_groupnorm_two_pass(op_engine, B, H, W, C1, C2, silu):
     test_groupnorm(op_engine, B, H, W, C1, C2, silu)
 
 
+@pytest.mark.parametrize("B,HW,C1,C2,G", [
+    (2, 13, 8, 0, 8),        # one octet, 512 pixel phases, 64 threads per group
+    (7, 72, 16, 0, 16),      # 32 threads per group
+    (3, 4, 8, 16, 8),        # fewer pixels than phases, a concat between groups
+    (1, 3053, 24, 0, 8),     # 3 channels per group
+    (2, 1001, 160, 0, 32),   # 5: the deal over 16 threads wraps inside a row
+    (1, 70001, 8, 0, 1),     # all channels one group, several rounds per thread
+    (2, 20011, 16, 0, 4),
+])
+def test_groupnorm_two_pass_groups(op_engine, B, HW, C1, C2, G):
+    """Few channels and other group counts on the statistics and apply passes, against fp64."""
+    say(f"groupnorm B={B} HW={HW} C1={C1} C2={C2} groups={G}")
+    e, C = op_engine, C1 + C2
+    x = r16((B, HW, C), 14, 2.0, 3.0)
+    g, b = r16((C,), 2, 0.3, 1.0), r16((C,), 3, 0.3)
+    ty = e.tensor((B, HW, C))
+    t2 = e.upload(x[:, :, C1:].astype(np.float16)) if C2 else None
+    names = kernels_of(e, lambda: e.groupnorm(e.upload(x[:, :, :C1].astype(np.float16)), e.upload(g.astype(np.float16)),
+                                              e.upload(b.astype(np.float16)), ty, B, HW, C1, C2, x2=t2, groups=G))
+    assert names == {"gn_stats_kernel", "gn_apply_kernel<0>"}
+    ref = torch.nn.functional.group_norm(t(x).double().transpose(1, 2), G, t(g).double(), t(b).double(), 1e-5)
+    ref = ref.transpose(1, 2).numpy()
+    got = ty.numpy().astype(np.float32)
+    assert rel_err_l1(got, ref) < 1e-3
+    assert np.abs(got - ref).max() < 2e-2
+
+
 def test_groupnorm_two_pass_large_mean(op_engine):
     """test_groupnorm_large_mean's bound for the statistics and apply passes (slabs of 92160 elements;
     3 channels per group)."""
