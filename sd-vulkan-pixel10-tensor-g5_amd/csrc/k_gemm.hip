@@ -1176,7 +1176,8 @@ hipError_t gemm_launch(GemmArgs a, float* ws, hipStream_t s) {
     const double kop = a.subpix ? 9.0 * a.Cin : (double)a.K;
     const double flops = 2.0 * a.M * a.N * kop;
     const double k_bytes = a_bytes + 2.0 * a.N * kop + out_bytes;
-    launch_timed(cfg_name(ci, a).c_str(), flops, k_bytes, [&] {
+    // (the name allocates: formed for a timer only)
+    launch_timed((g_kernel_timer ? cfg_name(ci, a) : std::string()).c_str(), flops, k_bytes, [&] {
         if (g.kind == K_PATCH) conv_patch_launch(g.shape, a, s);
         else if (g.kind == K_DENSE) dense_launch(g.shape, a, s);
         else if (a.amode == A_DENSE) launch_cfg<A_DENSE>(ci, grid, a, s);
