@@ -125,7 +125,10 @@ def taesd_engine():
     eng.release()
 
 
-@pytest.mark.parametrize("B,H,W", [(1, 16, 16), (2, 8, 12), (1, 64, 64)])
+@pytest.mark.parametrize("B,H,W", [
+    (1, 16, 16), (2, 8, 12), (1, 64, 64),
+    (1, 17, 23), (3, 19, 15),  # ragged tiles at every level; the upsampling convs in their 9-tap form
+])
 def test_taesd_decode_matches_oracle(taesd_engine, B, H, W):
     say(f"taesd decode B={B} {H}x{W}")
     z = (np.random.default_rng(B * 100 + H).standard_normal((B, 4, H, W)) * 1.5).astype(np.float32)
